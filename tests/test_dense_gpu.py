@@ -208,3 +208,57 @@ def test_the_dense_control_refuses_other_activation_dtypes(tn):
         tn._quantized_linear(xb, q)
     with pytest.raises(RuntimeError, match="mat1 and mat2 shapes cannot be multiplied"):
         tn._quantized_linear(_dev(tn, np.ones((2, 31), np.float32)), q)
+
+
+@pytest.mark.parametrize("m,k,n", [
+    # one row tile (16 x 64 per workgroup): fewer and one more than a stage of 64 k, the ring of six and past it
+    (1, 16, 1), (1, 60, 63), (16, 64, 64), (5, 68, 65), (16, 320, 64), (3, 384, 130), (16, 448, 17), (2, 1028, 70),
+    # 32 x 32: row and column remainders, the ring of five
+    (17, 16, 33), (32, 256, 32), (33, 336, 31), (200, 76, 96),
+    # 64 x 64 (512 workgroups)
+    (1024, 36, 2048), (1021, 144, 2049),
+    # rows that are no multiple of 16 bytes, and shorter than one product step
+    (4, 3, 9), (18, 15, 20), (16, 17, 16), (20, 131, 35), (7, 263, 50)])
+@pytest.mark.parametrize("fmt", ["f32", "f16", "bf16"])
+def test_linear_tiles_bit_for_bit(tn, m, k, n, fmt):
+    """Each tile shape of the dense linear at its edges, the oracle's fma chain
+    bit for bit, on operands that hold signed zeros, subnormals and values far
+    apart."""
+    rng = np.random.default_rng(m * 7 + k * 3 + n)
+
+    def operand(r):
+        a = np.ldexp(rng.standard_normal((r, k)), rng.integers(-12, 3, (r, k))).astype(np.float32)
+        a[rng.random((r, k)) < 0.1] = 0.0
+        a[rng.random((r, k)) < 0.1] = -0.0
+        tiny = rng.random((r, k)) < 0.05
+        a[tiny] = np.ldexp(rng.standard_normal(int(tiny.sum())), -140).astype(np.float32)
+        return a
+
+    x, w = operand(m), operand(n)
+    x[0] = 0.0  # a row of zeros, the sums' sign rules
+    b = rng.standard_normal(n).astype(np.float32) if n % 2 else None
+    q = tn._quantize(_dev(tn, w), fmt)
+    wide = tn._dequantize(q).numpy()
+    got = tn._quantized_linear(_dev(tn, x), q, None if b is None else _dev(tn, b)).numpy()
+    want = O.dense_linear(x, wide, b)
+    assert got.tobytes() == want.tobytes(), (m, k, n, fmt)
+
+
+@pytest.mark.parametrize("off", [1, 2])
+def test_linear_takes_rows_at_any_element(tn, off):
+    """Operands that start one or two elements past an aligned address (the
+    C ABI takes any pointer) give the aligned call's bits."""
+    from torchnative_amd import _lib
+
+    rng = np.random.default_rng(off)
+    m, k, n = 33, 64, 70
+    x = rng.standard_normal(m * k + 4).astype(np.float32)
+    w = rng.standard_normal(n * k + 8).astype(np.float32)
+    for fmt, code, es in (("f32", _lib.TN_F32, 4), ("f16", _lib.TN_F16, 2)):
+        xd, wd = _dev(tn, x), tn._quantize(_dev(tn, w.reshape(1, -1)), fmt)
+        wide = tn._dequantize(wd).numpy().reshape(-1)[off:off + n * k].reshape(n, k)
+        y = tn.empty((m, n), "float32", "hip")
+        _lib.check(_lib.lib().tn_dense_linear(None, xd.data_ptr() + 4 * off, m, k, wd._qs.data_ptr() + es * off, code, n,
+                                              None, y.data_ptr()))
+        want = O.dense_linear(x[off:off + m * k].reshape(m, k), wide, None)
+        assert y.numpy().tobytes() == want.tobytes(), fmt

@@ -184,6 +184,36 @@ __device__ inline void lds_direct16(buf_rsrc rsrc, uint32_t voffset, void* lds_w
 #endif
 }
 
+// lds_direct16 in assembly, for rings of many stages: the compiler neither
+// counts these loads nor takes LDS reads to depend on them, so the kernel
+// waits for a stage itself (wait_vmcnt, then a barrier) and no read waits for
+// the stages still in flight. Its own waits count only its own loads, which
+// can make them wait longer, never shorter. Offsets at or past `bytes` write
+// zeros.
+struct LdsDma {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    u4 rsrc;
+    __device__ LdsDma(const void* base, uint32_t bytes) {
+        const uint64_t a = reinterpret_cast<uint64_t>(base);
+        rsrc = (u4){(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xffffu)),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+    }
+    // lane l's 16 bytes at base + voffset go to lds + 16 l (lds wave-uniform)
+    __device__ __attribute__((always_inline)) inline void load16(uint32_t voffset, const void* lds) const {
+#if __HIP_DEVICE_COMPILE__
+        const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(m0), "v"(voffset), "s"(rsrc)
+                     : "memory");
+#else
+        (void)voffset, (void)lds;
+#endif
+    }
+};
+
 // v_max3_f32 (IEEE maxNum twice): written out because fmaxf on values the
 // compiler cannot prove quiet costs an extra canonicalising v_max per operand
 __device__ inline float max3f(float a, float b, float c) {
