@@ -110,6 +110,22 @@ tn_status workspace(hipStream_t stream, size_t bytes, void** out) {
     return TN_OK;
 }
 
+tn_status workspace_or_none(hipStream_t stream, size_t bytes, void** out) {
+    *out = nullptr;
+    int dev = 0;
+    TN_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        const Workspace& w = g_ws[{dev, stream}];
+        if (w.bytes < bytes) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            TN_HIP(hipStreamIsCapturing(stream, &cs));
+            if (cs != hipStreamCaptureStatusNone) return TN_OK;
+        }
+    }
+    return workspace(stream, bytes, out);
+}
+
 tn_status tickets(hipStream_t stream, size_t n, uint32_t** out) {
     int dev = 0;
     TN_HIP(hipGetDevice(&dev));

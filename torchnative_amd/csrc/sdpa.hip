@@ -32,6 +32,7 @@
 
 #include "tn_common.h"
 #include "attn_common.h"
+#include "flash_any.h"
 #include "skgeo.h"
 
 namespace tn {
@@ -1926,6 +1927,29 @@ tn_status static_scratch(hipStream_t, size_t bytes, void** out) {
 }
 }  // namespace
 
+// flash_any's view of a decode step: the nrep query heads of a key/value head
+// are its rows (consecutive in q, out and lse).
+static AnyArgs decode_any_args(const void* q, const void* k_cache, const void* v_cache, int64_t B, int64_t Hq,
+                               int64_t Hkv, int64_t cap, int64_t D, const int32_t* lens, int64_t max_len, double sc,
+                               void* out, float* lse) {
+    AnyArgs a{};
+    a.q = static_cast<const uint16_t*>(q);
+    a.k = static_cast<const uint16_t*>(k_cache);
+    a.v = static_cast<const uint16_t*>(v_cache);
+    a.out = static_cast<uint16_t*>(out);
+    a.lse = lse;
+    a.BH = (int)std::min<int64_t>(B * Hkv, INT32_MAX);  // flash_any_takes refuses the latter
+    a.Hq = a.Hkv = (int)Hkv;
+    a.L = (int)(Hq / Hkv);
+    a.S = (int)cap;
+    a.D = (int)D;
+    a.sl2 = (float)sc * LOG2E;
+    a.lens = lens;
+    a.max_len = (int)max_len;
+    a.nsplit = 1;
+    return a;
+}
+
 // Argument checks of the decode attention (shared with the decode step).
 tn_status decode_check(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t cap, int64_t D, int64_t max_len) {
     if (dtype != TN_BF16 && dtype != TN_F32 && dtype != TN_F16)
@@ -1952,6 +1976,36 @@ tn_status decode_check(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t ca
     return TN_OK;
 }
 
+// Decode attention at the head dims other than 64 and 128: flash_any for
+// 16-bit caches (the partials, if given, hold max_split splits of B * Hq
+// rows), otherwise the plain kernel, one query row per (sequence, head) over
+// the cache's cap rows.
+static tn_status decode_any(hipStream_t st, int dtype, const void* q, const void* k_cache, const void* v_cache, int64_t B,
+                            int64_t Hq, int64_t Hkv, int64_t cap, int64_t D, const int32_t* lens, int64_t max_len,
+                            double sc, void* out, float* lse, float* part_o, float2* part_ml, int max_split) {
+    if (dtype != TN_F32) {
+        AnyArgs a = decode_any_args(q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse);
+        if (flash_any_takes(a)) {
+            a.nsplit = part_o ? std::min(max_split, flash_any_splits(a)) : 1;
+            a.part_o = part_o;
+            a.part_ml = part_ml;
+            return flash_any_launch(st, dtype == TN_F16, a);
+        }
+    }
+    const dim3 grid(1u, (unsigned)Hq, (unsigned)B);
+    if (dtype == TN_F32)
+        hipLaunchKernelGGL((k_attn_any<0, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
+                           (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
+    else if (dtype == TN_BF16)
+        hipLaunchKernelGGL((k_attn_any<1, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
+                           (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
+    else
+        hipLaunchKernelGGL((k_attn_any<2, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
+                           (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
+    TN_LAUNCHED();
+    return TN_OK;
+}
+
 // Split-KV decode attention with caller-provided partial buffers (B*Hq*
 // ceil(max_len/256) rows of D floats, and as many (m, l) pairs): the grid is
 // sized by max_len, each workgroup reads its sequence's length on the device,
@@ -1963,23 +2017,9 @@ tn_status decode_launch(hipStream_t st, int dtype, const void* q, const void* k_
     const int nsplit = (int)cdiv(max_len, DEC_SPLIT);
     const double sc = std::isnan(scale) ? 1.0 / std::sqrt((double)D) : scale;
     const float sl2 = (float)sc * LOG2E;
-    if (D != 64 && D != 128) {
-        // the split kernels below exist for head dims 64 and 128; any other
-        // (up to 256, decode_check) runs on the plain kernel, one query row per
-        // (sequence, head) over the cache's cap rows, as tn_sdpa_decode does
-        const dim3 grid(1u, (unsigned)Hq, (unsigned)B);
-        if (dtype == TN_F32)
-            hipLaunchKernelGGL((k_attn_any<0, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        else if (dtype == TN_BF16)
-            hipLaunchKernelGGL((k_attn_any<1, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        else
-            hipLaunchKernelGGL((k_attn_any<2, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        TN_LAUNCHED();
-        return TN_OK;
-    }
+    if (D != 64 && D != 128)  // the split kernels below exist for head dims 64 and 128
+        return decode_any(st, dtype, q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse, part_o,
+                          part_ml, nsplit);
     if (dtype == TN_F32) {
         auto qq = static_cast<const float*>(q);
         auto kk = static_cast<const float*>(k_cache);
@@ -2316,6 +2356,42 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
     // scale >= 0) and exist for head dims 64 and 128; anything else runs on
     // the plain kernel
     if ((D != 64 && D != 128) || sc < 0.0 || dtype == TN_F64) {
+        if (dtype == TN_BF16 || dtype == TN_F16) {
+            AnyArgs a{};
+            a.q = static_cast<const uint16_t*>(q);
+            a.k = static_cast<const uint16_t*>(k);
+            a.v = static_cast<const uint16_t*>(v);
+            a.out = static_cast<uint16_t*>(out);
+            a.lse = lse;
+            a.BH = (int)std::min<int64_t>(B * Hq, INT32_MAX);  // flash_any_takes refuses the latter
+            a.Hq = (int)Hq;
+            a.Hkv = (int)Hkv;
+            a.L = (int)L;
+            a.S = (int)S;
+            a.D = (int)D;
+            a.sl2 = sl2;
+            a.causal = c;
+            a.nsplit = 1;
+            a.mk = mk;
+            a.mask = attn_mask;
+            a.msb = mref.sb, a.msh = mref.sh, a.msl = mref.sl, a.msk = mref.sk;
+            if (flash_any_takes(a)) {
+                const int ns = flash_any_splits(a);
+                if (ns > 1) {
+                    // split keys when the rows alone leave the device idle; under a
+                    // capture that could not grow the workspace, unsplit
+                    const size_t po = (size_t)rows * ns * D * sizeof(float), pm = (size_t)rows * ns * sizeof(float2);
+                    void* ws = nullptr;
+                    TN_TRY(workspace_or_none(st, po + pm, &ws));
+                    if (ws) {
+                        a.nsplit = ns;
+                        a.part_o = static_cast<float*>(ws);
+                        a.part_ml = reinterpret_cast<float2*>(static_cast<char*>(ws) + po);
+                    }
+                }
+                return flash_any_launch(st, dtype == TN_F16, a);
+            }
+        }
         const dim3 grid((unsigned)cdiv(L, ANY_BQ), (unsigned)Hq, (unsigned)B);
         const int et = dtype == TN_F32 ? 0 : dtype == TN_BF16 ? 1 : dtype == TN_F16 ? 2 : 3;
 #define TN_ANY(ET, MK)                                                                                            \
@@ -2480,21 +2556,26 @@ tn_status decode_entry(void* stream, int dtype, const void* q, const void* k_cac
         return fail(TN_EINVAL, "sdpa_decode: q, the caches and out must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
     if (D != 64 && D != 128) {
-        // the plain kernel: one query row per (sequence, head), the cache's cap
-        // rows as its keys, each sequence's length from lens
         const double sc = std::isnan(scale) ? 1.0 / std::sqrt((double)D) : scale;
-        const dim3 grid(1u, (unsigned)Hq, (unsigned)B);
-        if (dtype == TN_F32)
-            hipLaunchKernelGGL((k_attn_any<0, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        else if (dtype == TN_BF16)
-            hipLaunchKernelGGL((k_attn_any<1, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        else
-            hipLaunchKernelGGL((k_attn_any<2, 0>), grid, dim3(256), 0, st, q, k_cache, v_cache, (int)Hq, (int)Hkv, 1,
-                               (int)cap, (int)D, sc, 0, out, lse, MaskRef{}, lens, (int)max_len);
-        TN_LAUNCHED();
-        return TN_OK;
+        int ns = 1;
+        void* ws = nullptr;
+        size_t po = 0;
+        if (dtype != TN_F32) {
+            const AnyArgs a = decode_any_args(q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse);
+            if (flash_any_takes(a)) ns = flash_any_splits(a);
+            if (ns > 1) {
+                // as many splits as the no-alloc entry's array holds, in either
+                // entry (they give the same bits); none where a capture could not
+                // grow the stream's workspace
+                const size_t one = (size_t)B * Hq * (D * sizeof(float) + sizeof(float2));
+                ns = (int)std::min<size_t>(ns, DECODE_SCRATCH_BYTES / one);
+                po = (size_t)B * Hq * ns * D * sizeof(float);
+                if (ns > 1) TN_TRY((get == workspace ? workspace_or_none : get)(st, one * ns, &ws));
+            }
+        }
+        return decode_any(st, dtype, q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse,
+                          static_cast<float*>(ws), ws ? reinterpret_cast<float2*>(static_cast<char*>(ws) + po) : nullptr,
+                          ns);
     }
     // the stream-K kernel counts 16-key units of all segments in an int
     const bool half = dtype == TN_BF16 || dtype == TN_F16;

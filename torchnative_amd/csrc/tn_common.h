@@ -33,6 +33,9 @@ Counters& counters();
 // Grow-only device workspace, one per (device, stream). Calls on one stream
 // are ordered, so reuse across them is safe.
 tn_status workspace(hipStream_t stream, size_t bytes, void** out);
+// The same for a call that can do without: null, and no refusal, where the
+// stream is under graph capture and its workspace would have to grow.
+tn_status workspace_or_none(hipStream_t stream, size_t bytes, void** out);
 // Per-(device, stream) array of n uint32 counters, zero when first handed out
 // (cleared on the stream at allocation). A kernel that takes tickets from it
 // must leave every counter at zero again when it ends.
