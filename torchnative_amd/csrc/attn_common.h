@@ -212,6 +212,19 @@ struct LdsDma {
         (void)voffset, (void)lds;
 #endif
     }
+    // lane l's 2 bytes, zero-extended, go to the dword lds + 4 l
+    __device__ __attribute__((always_inline)) inline void load2(uint32_t voffset, const void* lds) const {
+#if __HIP_DEVICE_COMPILE__
+        const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane(
+            (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_ushort %1, %2, 0 offen lds"
+                     :
+                     : "s"(m0), "v"(voffset), "s"(rsrc)
+                     : "memory");
+#else
+        (void)voffset, (void)lds;
+#endif
+    }
 };
 
 // v_max3_f32 (IEEE maxNum twice): written out because fmaxf on values the

@@ -1,6 +1,6 @@
 // GGML block-quantised weights on gfx950 (q4_0 and q8_0): upload/repack,
-// quantise, dequantise, and the quantised linear (decode GEMV and prefill
-// MFMA GEMM).
+// quantise, dequantise, and the quantised linear (the decode GEMV here; more
+// rows on qgemm.hip).
 //
 // Arithmetic contract (candle-core/src/quantized/k_quants.rs, the reference's
 // vendored candle): every output is
@@ -13,17 +13,15 @@
 // below performs the float steps in exactly that order with separate
 // roundings (the library is built with -ffp-contract=off), so results are
 // bit-identical to the reference's x86_64 scalar path for every row count.
-#include "tn_common.h"
+#include "q8.h"
+#include "qgemm.h"
 
 namespace tn {
 namespace {
 
-constexpr int QK = 32;
-
 // Weight formats. On the device a weight is two planes: the codes of every
 // block back to back in row-major block order (q4_0: the 16 nibble bytes of
 // the GGML block; q8_0: its 32 int8 codes) and the f16 block scales.
-enum WeightFormat { FMT_Q4_0 = 0, FMT_Q8_0 = 1 };
 template <int FMT>
 struct Fmt;
 template <>
@@ -38,44 +36,6 @@ struct Fmt<FMT_Q8_0> {
     static constexpr int GEMV_ITEMS = 3;  // 32-byte items: 96 bytes in flight per thread (5.40 TB/s at the C1 shape; 5.12 for 2, 5.34 for 4)
     static constexpr const char* name = "q8_0";
 };
-
-// ---- Rust cast semantics ---------------------------------------------------
-
-// Truncation toward zero after clamping to the type's range, NaN to 0. The
-// clamp and the NaN test are selects: written as early returns they became
-// three nested exec-mask branches per element.
-__device__ inline int sat_i8(float v) {  // `f as i8`
-    const int q = (int)fminf(fmaxf(v, -128.0f), 127.0f);
-    return v != v ? 0 : q;
-}
-
-__device__ inline int sat_u8(float v) {  // `f as u8`
-    const int q = (int)fminf(fmaxf(v, 0.0f), 255.0f);
-    return v != v ? 0 : q;
-}
-
-template <typename XT>
-__device__ inline float load_x(const XT* p);
-template <>
-__device__ inline float load_x<float>(const float* p) { return *p; }
-template <>
-__device__ inline float load_x<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
-
-// Q8_0 of one 32-element block held one element per lane of a 32-lane group
-// (BlockQ8_0::from_float, k_quants.rs:676-705): amax over the block, d =
-// amax/127 (IEEE division), id = 1/d or 0, q = (round-half-away(x*id)) as i8.
-// Returns q; *dx gets f32(f16(d)), the scale the dot product uses.
-__device__ inline int q8_0_lane(float v, float* dx) {
-    // f32::max from 0 (k_quants.rs:676-705): a NaN lane counts as 0, so a
-    // block of NaNs has amax 0, id 0 and zero codes, as the reference's has
-    float a = fmaxf(0.0f, fabsf(v));
-#pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 32));
-    float d = a / 127.0f;
-    float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-    *dx = f16_to_f32(f16_from_f32(d));
-    return sat_i8(roundf(v * id));
-}
 
 // ---- layout conversion --------------------------------------------------------
 
@@ -810,606 +770,6 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_gemv(const XT* __restrict__ x,
     if constexpr (ARG) gemv_argmax_epilogue(best_v, best_i, po);
 }
 
-// ---- prefill GEMM on MFMA ---------------------------------------------------------
-//
-// Prepass: every activation row is quantised to Q8_0 once, into bf16 codes
-// (|q| <= 127 is exact in bf16) laid out per block in the order the MFMA
-// operand wants, plus the f32 block scales transposed [nb][M_pad].
-//
-// Main kernel: a 128x128 output tile per workgroup, four waves as 2x2, each
-// wave 64x64 = 4x4 tiles of v_mfma_f32_16x16x32_bf16. The K loop walks blocks
-// in order, double-buffered in LDS: the next block's loads are issued into
-// registers before the current block is computed.
-//
-// Exactness. The weight codes enter the MFMA as bf16(128 + nib), built by one
-// byte permute per two nibbles (the bf16 bit pattern of 128 + n is 0x4300 | n),
-// and the accumulator starts at -136 * sum_j(x codes) for the row, so the MFMA
-// returns sum_j (nib_j - 8) * q_j = the block's integer dot S_b exactly: every
-// product (<= 143*127), every partial sum and the start value stay below 2^24
-// in magnitude, so no fp32 step rounds. S_b then gets the reference's two
-// roundings, (S_b * d_w) * d_x, and one addition into the running sum, in
-// block order.
-//
-// K-slot order: MFMA lane group g (lanes 16g..16g+15) holds 8 of the 32 block
-// elements, {4g..4g+3, 16+4g..16+4g+3}: the low and high nibbles of weight
-// bytes 4g..4g+3. The activation codes are stored in the same order, so the
-// two operands agree element for element.
-//
-// Tile order is XCD-aware: consecutive workgroups go to different XCDs, so the
-// workgroup index is remapped such that each XCD works on a contiguous range
-// of weight columns and reads those columns into its own L2 once for all the
-// row tiles.
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int GM_BM = 128, GM_BN = 128, GM_THREADS = 256;
-constexpr int NUM_XCD = 8;
-
-__device__ inline int kslot_of_element(int e) {  // element (0..31) -> K slot
-    return e < 16 ? 8 * (e >> 2) + (e & 3) : 8 * ((e - 16) >> 2) + 4 + (e & 3);
-}
-
-template <typename XT>
-__global__ __launch_bounds__(256) void k_q8_rows(const XT* __restrict__ x, int M, int M_pad, int K, int nb,
-                                               uint16_t* __restrict__ xc, float* __restrict__ dxT,
-                                               float* __restrict__ corrT) {
-    // one 32-lane group per (row, block); rows >= M become zero codes, zero scale
-    const int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 5) + (threadIdx.x >> 5);
-    const int lane = threadIdx.x & 31;
-    if (blk >= (int64_t)M_pad * nb) return;
-    const int row = (int)(blk / nb), b = (int)(blk - (int64_t)row * nb);
-    float dx = 0.0f;
-    int q = 0;
-    if (row < M) {
-        float v = load_x<XT>(x + (int64_t)row * K + b * QK + lane);
-        q = q8_0_lane(v, &dx);
-    }
-    int s = q;
-#pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) s += __shfl_xor(s, off, 32);
-    xc[blk * QK + kslot_of_element(lane)] = (uint16_t)(__builtin_bit_cast(uint32_t, (float)q) >> 16);
-    if (lane == 0) {
-        dxT[(int64_t)b * M_pad + row] = dx;
-        corrT[(int64_t)b * M_pad + row] = (float)(-136 * s);
-    }
-}
-
-// Eight consecutive activations as floats: 16 bytes of bf16 or 32 of f32
-// (p 16-byte aligned).
-template <typename XT>
-__device__ inline void load_x8(const XT* p, float (&v)[8]);
-template <>
-__device__ inline void load_x8<float>(const float* p, float (&v)[8]) {
-    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-}
-template <>
-__device__ inline void load_x8<uint16_t>(const uint16_t* p, float (&v)[8]) {
-    const uint4 a = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        v[2 * i] = __builtin_bit_cast(float, w[i] << 16);
-        v[2 * i + 1] = __builtin_bit_cast(float, w[i] & 0xffff0000u);
-    }
-}
-
-// The Q8_0 codes of one block held by four lanes, eight elements each: the
-// block's amax (order-free), d = amax/127, id = 1/d and the rounding are
-// q8_0_lane's, element for element, so the codes, the scale and the code sum
-// are identical; the sum comes back through `s`.
-__device__ inline void q8_0_quad(const float (&v)[8], int (&q)[8], float* dx, int* s) {
-    float a = 0.0f;  // f32::max from 0: NaNs are skipped (k_quants.rs:676-705)
-#pragma unroll
-    for (int e = 0; e < 8; e++) a = fmaxf(a, fabsf(v[e]));
-    a = fmaxf(a, __shfl_xor(a, 1, 4));
-    a = fmaxf(a, __shfl_xor(a, 2, 4));
-    const float d = a / 127.0f;
-    const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-    *dx = f16_to_f32(f16_from_f32(d));
-    int sum = 0;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        q[e] = sat_i8(roundf(v[e] * id));
-        sum += q[e];
-    }
-    sum += __shfl_xor(sum, 1, 4);
-    sum += __shfl_xor(sum, 2, 4);
-    *s = sum;
-}
-
-// How the prepass finds a row's activations (XM_* in tn_common.h). XM_ROWS:
-// row r is x[r][0..K). XM_GLU: x holds [M][2K] rows (gate | up) and the
-// activation is silu(gate) * up, k_silu_mul's arithmetic (decode.hip).
-// XM_HEADS: x is an attention output [K / hd][M][hd] (head-major) and row r
-// is its heads' rows of token r side by side. The last two let a prompt's
-// down and o projections read their producers' outputs without a copy in
-// between.
-
-// k_q8_rows for a 16-byte aligned x: four lanes per (row, block), one 16- or
-// 32-byte load each. Lane part p holds elements 8p .. 8p+7, whose K slots are
-// two runs of four (kslot_of_element), written as two 8-byte stores.
-template <typename XT, int XM = XM_ROWS>
-__global__ __launch_bounds__(256) void k_q8_rows_v(const XT* __restrict__ x, int M, int M_pad, int K, int nb,
-                                                   uint16_t* __restrict__ xc, float* __restrict__ dxT,
-                                                   float* __restrict__ corrT, int hd = 0) {
-    const int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2);
-    const int part = threadIdx.x & 3;
-    if (blk >= (int64_t)M_pad * nb) return;  // the four lanes of a block leave together
-    const int row = (int)(blk / nb), b = (int)(blk - (int64_t)row * nb);
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (row < M) {
-        if constexpr (XM == XM_GLU) {
-            float g[8], u[8];
-            load_x8<XT>(x + (int64_t)row * 2 * K + b * QK + 8 * part, g);
-            load_x8<XT>(x + (int64_t)row * 2 * K + K + b * QK + 8 * part, u);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = (g[e] / (1.0f + expf(-g[e]))) * u[e];
-        } else if constexpr (XM == XM_HEADS) {
-            const int e0 = b * QK, h = e0 / hd;
-            load_x8<XT>(x + ((int64_t)h * M + row) * hd + (e0 - h * hd) + 8 * part, v);
-        } else {
-            load_x8<XT>(x + (int64_t)row * K + b * QK + 8 * part, v);
-        }
-    }
-    int q[8], s;
-    float dx;
-    q8_0_quad(v, q, &dx, &s);
-    if (row >= M) dx = 0.0f;
-    auto code = [](int c) { return __builtin_bit_cast(uint32_t, (float)c) >> 16; };
-    const int slot0 = kslot_of_element(8 * part), slot1 = kslot_of_element(8 * part + 4);
-    *reinterpret_cast<uint2*>(xc + blk * QK + slot0) =
-        make_uint2(code(q[0]) | (code(q[1]) << 16), code(q[2]) | (code(q[3]) << 16));
-    *reinterpret_cast<uint2*>(xc + blk * QK + slot1) =
-        make_uint2(code(q[4]) | (code(q[5]) << 16), code(q[6]) | (code(q[7]) << 16));
-    if (part == 0) {
-        dxT[(int64_t)b * M_pad + row] = dx;
-        corrT[(int64_t)b * M_pad + row] = (float)(-136 * s);
-    }
-}
-
-// bytes 0,1 (or 2,3) of x -> the bf16 pair (128 + byte0, 128 + byte1): the
-// high byte of each half comes from the constant 0x43
-__device__ inline uint32_t codes_pair01(uint32_t x) { return __builtin_amdgcn_perm(0x43434343u, x, 0x04010400u); }
-__device__ inline uint32_t codes_pair23(uint32_t x) { return __builtin_amdgcn_perm(0x43434343u, x, 0x04030402u); }
-
-constexpr int GM_AS = QK + 8;  // LDS row stride (bf16) of the code tiles: 80 B, conflict-free b128 reads
-constexpr int GM_RS = 4;       // K blocks whose operands are in flight ahead of the one computed
-
-// WR x WC waves over a GM_BM x BN tile, each wave TI x TJ MFMA tiles of
-// 16x16: <2, 2, 4> is 128 x 128 (waves of 64 x 64), <4, 1, 7> is 128 x 112
-// (waves of 32 x 112), chosen at launch so the tiles fill the device evenly.
-// Products with few rows and columns (a prompt's projections) take narrow
-// tiles, <4, 1, TJ> with 16 TJ columns, so that more workgroups share the
-// work: each walks every K block in order whatever its tile, so the number
-// of workgroups, not their width, sets such a call's time.
-template <int WR, int WC, int TJ>
-__global__ __launch_bounds__(GM_THREADS) void k_gemm(const uint16_t* __restrict__ xc,
-                                                    const float* __restrict__ dxT,
-                                                    const float* __restrict__ corrT, int M, int M_pad, int nb,
-                                                    const uint8_t* __restrict__ qs,
-                                                    const uint16_t* __restrict__ dw, int N,
-                                                    const float* __restrict__ bias, void* y, int y_bf16,
-                                                    const float* resid = nullptr) {
-    static_assert(WR * WC == GM_THREADS / 64, "one wave per sub-tile");
-    constexpr int TI = GM_BM / (16 * WR);  // MFMA row tiles per wave
-    constexpr int BN = 16 * TJ * WC;       // columns per workgroup
-    static_assert(2 * BN <= GM_THREADS && GM_BM + BN <= GM_THREADS, "staging threads");
-    __shared__ __align__(16) uint16_t sA[2][GM_BM * GM_AS];
-    __shared__ __align__(16) uint16_t sB[2][BN * GM_AS];
-    __shared__ __align__(16) float sdx[2][GM_BM];
-    __shared__ __align__(16) float scr[2][GM_BM];
-    __shared__ __align__(16) float sdw[2][BN];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / WC, wn = wave % WC;  // wave's (16 TI) x (16 TJ) sub-tile
-    const int lrow = lane & 15, lgrp = lane >> 4;
-
-    // XCD-aware tile order: workgroup id -> (row tile, column tile)
-    const int mt = (int)gridDim.y;              // row tiles
-    const int ntot = (int)(gridDim.x * gridDim.y);
-    const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-    int tile = id;
-    if (ntot % NUM_XCD == 0) tile = (id % NUM_XCD) * (ntot / NUM_XCD) + id / NUM_XCD;
-    const int m0 = (tile % mt) * GM_BM, n0 = (tile / mt) * BN;
-
-    f32x4 acc[TI][TJ];
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int j = 0; j < TJ; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // Per-thread staging registers, GM_RS register sets: block b's operands are
-    // requested GM_RS blocks before they are computed (about 1.7 us of
-    // memory latency against about 0.4 us of work per block), then stored to
-    // the LDS double buffer one block ahead. The set index is a compile-time
-    // constant (the K loop is unrolled by GM_RS), so the sets stay in VGPRs.
-    // one register set: two 16-byte chunks of activation codes, 8 bytes of
-    // weight nibbles (threads < 2 BN), and (threads < GM_BM) the row's Q8_0
-    // scale and accumulator start or (GM_BM <= threads < GM_BM + BN) the
-    // column's f16 weight scale
-    const int bcol = tid >> 1, bhalf = tid & 1;
-    const int ar0 = tid >> 2, ar1 = (tid + GM_THREADS) >> 2, apart = tid & 3;  // the two A chunks
-    // Every load is an unconditional buffer load: a descriptor per operand
-    // over this tile's rows or columns, a per-thread offset computed once and
-    // the block's offset in a scalar register, so a step costs no address
-    // arithmetic. What lies past a descriptor's range (columns past N, the
-    // threads that stage nothing of an operand, blocks past the last) reads
-    // as zero and is not used; loads behind branches made the compiler's wait
-    // counting fall back to waiting for every load in flight.
-    const uint32_t OOB = 0x80000000u;  // an offset past every range here
-    const int ncols = min(BN, N - n0);
-    const buf_rsrc ra = make_rsrc(xc + (int64_t)m0 * nb * QK, (uint32_t)(GM_BM * nb * QK * 2));
-    const buf_rsrc rw = make_rsrc(qs + (int64_t)n0 * nb * 16, (uint32_t)(ncols * nb * 16));
-    const buf_rsrc rdx = make_rsrc(dxT + m0, (uint32_t)(((int64_t)nb * M_pad - m0) * 4));
-    const buf_rsrc rcr = make_rsrc(corrT + m0, (uint32_t)(((int64_t)nb * M_pad - m0) * 4));
-    const buf_rsrc rdw = make_rsrc(dw + (int64_t)n0 * nb, (uint32_t)(ncols * nb * 2));
-    const uint32_t va0 = (uint32_t)((ar0 * nb * QK + apart * 8) * 2), va1 = (uint32_t)((ar1 * nb * QK + apart * 8) * 2);
-    const uint32_t vw = bcol < BN ? (uint32_t)(bcol * nb * 16 + bhalf * 8) : OOB;
-    const uint32_t vs = tid < GM_BM ? (uint32_t)(tid * 4) : OOB;
-    const uint32_t vd = (tid >= GM_BM && tid < GM_BM + BN) ? (uint32_t)((tid - GM_BM) * nb * 2) : OOB;
-    auto gload = [&](int b, uint4& a0, uint4& a1, uint2& w, float& dx, float& corr, uint32_t& dws)
-                     __attribute__((always_inline)) {
-        // Blocks past the last (the prefetches of the final steps, and the
-        // first four when nb < 4) are clamped to the last block. The block
-        // offset travels in the scalar offset, which the descriptor's range
-        // check does not cover, so it must itself stay inside the operands.
-        // The clamped data lands in an LDS buffer no later step reads.
-        b = min(b, nb - 1);
-#if __HIP_DEVICE_COMPILE__
-        typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-        typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-        const u32x4_t x0 = __builtin_amdgcn_raw_buffer_load_b128(ra, va0, (uint32_t)(b * QK * 2), 0);
-        const u32x4_t x1 = __builtin_amdgcn_raw_buffer_load_b128(ra, va1, (uint32_t)(b * QK * 2), 0);
-        const u32x2_t ww = __builtin_amdgcn_raw_buffer_load_b64(rw, vw, (uint32_t)(b * 16), 0);
-        a0 = make_uint4(x0[0], x0[1], x0[2], x0[3]);
-        a1 = make_uint4(x1[0], x1[1], x1[2], x1[3]);
-        w = make_uint2(ww[0], ww[1]);
-        dx = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rdx, vs, (uint32_t)(b * M_pad * 4), 0));
-        corr = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rcr, vs, (uint32_t)(b * M_pad * 4), 0));
-        dws = __builtin_amdgcn_raw_buffer_load_b16(rdw, vd, (uint32_t)(b * 2), 0);
-#else
-        (void)b;
-        a0 = a1 = make_uint4(0, 0, 0, 0);
-        w = make_uint2(0, 0);
-        dx = corr = 0.0f;
-        dws = 0;
-#endif
-    };
-    auto lstore = [&](int buf, const uint4& a0, const uint4& a1, const uint2& w, float dx, float corr,
-                      uint32_t dws) __attribute__((always_inline)) {
-        *reinterpret_cast<uint4*>(&sA[buf][ar0 * GM_AS + apart * 8]) = a0;
-        *reinterpret_cast<uint4*>(&sA[buf][ar1 * GM_AS + apart * 8]) = a1;
-        // weight dwords g = 2*bhalf, 2*bhalf+1 -> K slots 8g..8g+7 each
-        const uint32_t w0 = w.x, w1 = w.y;
-        const uint32_t lo0 = w0 & 0x0f0f0f0fu, hi0 = (w0 >> 4) & 0x0f0f0f0fu;
-        const uint32_t lo1 = w1 & 0x0f0f0f0fu, hi1 = (w1 >> 4) & 0x0f0f0f0fu;
-        if (bcol < BN) {
-            uint4* dst = reinterpret_cast<uint4*>(&sB[buf][bcol * GM_AS + bhalf * 16]);
-            dst[0] = make_uint4(codes_pair01(lo0), codes_pair23(lo0), codes_pair01(hi0), codes_pair23(hi0));
-            dst[1] = make_uint4(codes_pair01(lo1), codes_pair23(lo1), codes_pair01(hi1), codes_pair23(hi1));
-        }
-        if (tid < GM_BM) {
-            sdx[buf][tid] = dx;
-            scr[buf][tid] = corr;
-        } else if (tid < GM_BM + BN) {
-            sdw[buf][tid - GM_BM] = f16_bits_hw((uint16_t)dws);
-        }
-    };
-    // one K block from LDS buffer `buf`: the exact block dot on MFMA, then
-    // the reference's two roundings and the ordered addition
-    auto compute = [&](int buf) __attribute__((always_inline)) {
-        constexpr int WROWS = 16 * TI, WCOLS = 16 * TJ;  // the wave's sub-tile
-        bf16x8 afr[TI], bfr[TJ];
-#pragma unroll
-        for (int i = 0; i < TI; i++)
-            afr[i] = *reinterpret_cast<const bf16x8*>(&sA[buf][(wm * WROWS + i * 16 + lrow) * GM_AS + lgrp * 8]);
-#pragma unroll
-        for (int j = 0; j < TJ; j++)
-            bfr[j] = *reinterpret_cast<const bf16x8*>(&sB[buf][(wn * WCOLS + j * 16 + lrow) * GM_AS + lgrp * 8]);
-        float dwv[TJ];
-        f32x4 dxv[TI], crv[TI];
-#pragma unroll
-        for (int j = 0; j < TJ; j++) dwv[j] = sdw[buf][wn * WCOLS + j * 16 + lrow];
-#pragma unroll
-        for (int i = 0; i < TI; i++) {
-            dxv[i] = *reinterpret_cast<const f32x4*>(&sdx[buf][wm * WROWS + i * 16 + lgrp * 4]);
-            crv[i] = *reinterpret_cast<const f32x4*>(&scr[buf][wm * WROWS + i * 16 + lgrp * 4]);
-        }
-        // C[row][col]: col = lane & 15 (weight column), row = 4*(lane>>4) + r;
-        // A = activation rows, B = weight columns; C starts at -136*sum(x codes).
-        // Tile k + 1's product is issued before tile k's recurrence, in that
-        // order (the scheduling barriers pin it), so each product runs on the
-        // matrix core under the previous tile's VALU work.
-        constexpr int NT = TI * TJ;
-        f32x4 sv[2];
-        sv[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr[0], bfr[0], crv[0], 0, 0, 0);
-#pragma unroll
-        for (int k = 0; k < NT; k++) {
-            const int i = k / TJ, j = k % TJ;
-            if (k + 1 < NT) {
-                const int i1 = (k + 1) / TJ, j1 = (k + 1) % TJ;
-                __builtin_amdgcn_sched_barrier(0);
-                sv[(k + 1) & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr[i1], bfr[j1], crv[i1], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                float t = sv[k & 1][r] * dwv[j];
-                t = t * dxv[i][r];
-                acc[i][j][r] = acc[i][j][r] + t;
-            }
-        }
-        // the block's additions are done here, before the step's barrier: left
-        // to itself the compiler sinks them past the next steps' products and
-        // holds several blocks' products in registers at once
-#pragma unroll
-        for (int i = 0; i < TI; i++)
-#pragma unroll
-            for (int j = 0; j < TJ; j++) asm volatile("" : "+v"(acc[i][j]));
-    };
-    // Four register sets, named: step b refills set b % 4 with block b + 4
-    // (set b's data went to LDS at the end of step b - 1), computes block b,
-    // and stores block b + 1 to the other LDS buffer.
-    uint4 a0_0, a1_0, a0_1, a1_1, a0_2, a1_2, a0_3, a1_3;
-    uint2 w_0, w_1, w_2, w_3;
-    float dx_0, dx_1, dx_2, dx_3, cr_0, cr_1, cr_2, cr_3;
-    uint32_t dw_0, dw_1, dw_2, dw_3;
-    static_assert(GM_RS == 4, "the unrolled K loop below names four register sets");
-#define TN_GM_SET(S) a0_##S, a1_##S, w_##S, dx_##S, cr_##S, dw_##S
-    // (the last steps load and stage a block past the end, clamped by gload
-    // to the last one, into the LDS buffer no later step reads)
-#define TN_GM_STEP(S, NEXT, B)                          \
-    {                                                   \
-        gload((B) + GM_RS, TN_GM_SET(S));               \
-        compute((B)&1);                                 \
-        lstore(((B) + 1) & 1, TN_GM_SET(NEXT));         \
-        __syncthreads();                                \
-    }
-    gload(0, TN_GM_SET(0));
-    gload(1, TN_GM_SET(1));
-    gload(2, TN_GM_SET(2));
-    gload(3, TN_GM_SET(3));
-    lstore(0, TN_GM_SET(0));
-    __syncthreads();
-    // whole rounds of four steps as straight-line code, then the rest
-    int b = 0;
-    for (; b + GM_RS <= nb; b += GM_RS) {
-        TN_GM_STEP(0, 1, b)
-        TN_GM_STEP(1, 2, b + 1)
-        TN_GM_STEP(2, 3, b + 2)
-        TN_GM_STEP(3, 0, b + 3)
-    }
-    if (b < nb) TN_GM_STEP(0, 1, b)
-    if (b + 1 < nb) TN_GM_STEP(1, 2, b + 1)
-    if (b + 2 < nb) TN_GM_STEP(2, 3, b + 2)
-#undef TN_GM_STEP
-#undef TN_GM_SET
-
-#pragma unroll
-    for (int i = 0; i < TI; i++) {
-#pragma unroll
-        for (int j = 0; j < TJ; j++) {
-            const int n = n0 + wn * 16 * TJ + j * 16 + lrow;
-            if (n >= N) continue;
-            const float bv = bias ? bias[n] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 16 * TI + i * 16 + lgrp * 4 + r;
-                if (m >= M) continue;
-                float v = acc[i][j][r];
-                if (bias) v = v + bv;
-                // resid + y, tn_add's operation, into y (f32); resid may be y
-                if (resid) v = resid[(int64_t)m * N + n] + v;
-                if (y_bf16)
-                    reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = bf16_from_f32(v);
-                else
-                    reinterpret_cast<float*>(y)[(int64_t)m * N + n] = v;
-            }
-        }
-    }
-}
-
-
-// ---- q8_0 prefill GEMM on integer MFMA -----------------------------------------
-//
-// With q8_0 weights both operands are int8 codes, so the block dot S_b is one
-// v_mfma_i32_16x16x32_i8 per 16x16 output tile and K block: an exact i32
-// result with no offset correction and no code conversion. The tile shape,
-// the XCD-aware tile order, the LDS double buffer and the four register sets
-// in flight are k_gemm's; the float steps are the same (S_b * d_w) * d_x and
-// ordered addition.
-//
-// Prepass: the activation rows' Q8_0 codes as int8 in natural element order
-// ([M_pad][nb][32]) and the f32 block scales transposed [nb][M_pad].
-//
-// LDS holds each 128 x 32-byte operand tile in MFMA fragment order: for row
-// tile t (16 rows) and lane group g, the 16 rows' bytes 8g..8g+7 are 128
-// consecutive bytes, so a fragment read is one conflict-free ds_read_b64 of
-// 512 contiguous bytes per wave. Lane l of the MFMA holds row l % 16, block
-// elements 8 (l / 16) .. 8 (l / 16) + 7 of both operands.
-
-template <typename XT>
-__global__ __launch_bounds__(256) void k_q8_rows_i8(const XT* __restrict__ x, int M, int M_pad, int K, int nb,
-                                                   int8_t* __restrict__ xc, float* __restrict__ dxT) {
-    // one 32-lane group per (row, block); rows >= M become zero codes, zero scale
-    const int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 5) + (threadIdx.x >> 5);
-    const int lane = threadIdx.x & 31;
-    if (blk >= (int64_t)M_pad * nb) return;
-    const int row = (int)(blk / nb), b = (int)(blk - (int64_t)row * nb);
-    float dx = 0.0f;
-    int q = 0;
-    if (row < M) {
-        float v = load_x<XT>(x + (int64_t)row * K + b * QK + lane);
-        q = q8_0_lane(v, &dx);
-    }
-    xc[blk * QK + lane] = (int8_t)q;
-    if (lane == 0) dxT[(int64_t)b * M_pad + row] = dx;
-}
-
-// k_q8_rows_i8 for a 16-byte aligned x: four lanes per (row, block), eight
-// int8 codes each in natural order (one 8-byte store).
-template <typename XT>
-__global__ __launch_bounds__(256) void k_q8_rows_i8_v(const XT* __restrict__ x, int M, int M_pad, int K, int nb,
-                                                      int8_t* __restrict__ xc, float* __restrict__ dxT) {
-    const int64_t blk = (int64_t)blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2);
-    const int part = threadIdx.x & 3;
-    if (blk >= (int64_t)M_pad * nb) return;
-    const int row = (int)(blk / nb), b = (int)(blk - (int64_t)row * nb);
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (row < M) load_x8<XT>(x + (int64_t)row * K + b * QK + 8 * part, v);
-    int q[8], s;
-    float dx;
-    q8_0_quad(v, q, &dx, &s);
-    if (row >= M) dx = 0.0f;
-    uint32_t w[2] = {0u, 0u};
-#pragma unroll
-    for (int e = 0; e < 8; e++) w[e >> 2] |= ((uint32_t)q[e] & 0xffu) << (8 * (e & 3));
-    *reinterpret_cast<uint2*>(xc + blk * QK + 8 * part) = make_uint2(w[0], w[1]);
-    if (part == 0) dxT[(int64_t)b * M_pad + row] = dx;
-}
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-__device__ inline int frag_offset(int r, int g) {  // byte offset of row r, bytes 8g..8g+7, in a fragment-ordered tile
-    return ((r >> 4) * 4 + g) * 128 + (r & 15) * 8;
-}
-
-__global__ __launch_bounds__(GM_THREADS) void k_gemm_q8(const int8_t* __restrict__ xc, const float* __restrict__ dxT,
-                                                       int M, int M_pad, int nb, const uint8_t* __restrict__ qs,
-                                                       const uint16_t* __restrict__ dw, int N,
-                                                       const float* __restrict__ bias, void* __restrict__ y,
-                                                       int y_bf16) {
-    __shared__ __align__(16) uint8_t sA[2][GM_BM * QK];
-    __shared__ __align__(16) uint8_t sB[2][GM_BN * QK];
-    __shared__ __align__(16) float sdx[2][GM_BM];
-    __shared__ __align__(16) float sdw[2][GM_BN];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;  // wave's 64x64 sub-tile
-    const int lrow = lane & 15, lgrp = lane >> 4;
-
-    const int mt = (int)gridDim.y;
-    const int ntot = (int)(gridDim.x * gridDim.y);
-    const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-    int tile = id;
-    if (ntot % NUM_XCD == 0) tile = (id % NUM_XCD) * (ntot / NUM_XCD) + id / NUM_XCD;
-    const int m0 = (tile % mt) * GM_BM, n0 = (tile / mt) * GM_BN;
-
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // one register set: 16 bytes of activation codes (row tid / 2, half tid % 2),
-    // 16 bytes of weight codes (column tid / 2), and (threads < GM_BM) the
-    // row's Q8_0 scale or (threads >= GM_BM) the column's f16 weight scale
-    const int prow = tid >> 1, phalf = tid & 1;
-    const int so0 = frag_offset(prow, 2 * phalf), so1 = frag_offset(prow, 2 * phalf + 1);
-    auto gload = [&](int b, uint4& a, uint4& w, float& dx, uint32_t& dws) {
-        a = *reinterpret_cast<const uint4*>(xc + ((int64_t)(m0 + prow) * nb + b) * QK + phalf * 16);
-        w = make_uint4(0u, 0u, 0u, 0u);
-        if (n0 + prow < N) w = *reinterpret_cast<const uint4*>(qs + ((int64_t)(n0 + prow) * nb + b) * QK + phalf * 16);
-        dx = 0.0f;
-        dws = 0;
-        if (tid < GM_BM) {
-            dx = dxT[(int64_t)b * M_pad + m0 + tid];
-        } else {
-            const int n = n0 + tid - GM_BM;
-            dws = (n < N) ? dw[(int64_t)n * nb + b] : 0u;
-        }
-    };
-    auto lstore = [&](int buf, const uint4& a, const uint4& w, float dx, uint32_t dws) {
-        *reinterpret_cast<uint2*>(&sA[buf][so0]) = make_uint2(a.x, a.y);
-        *reinterpret_cast<uint2*>(&sA[buf][so1]) = make_uint2(a.z, a.w);
-        *reinterpret_cast<uint2*>(&sB[buf][so0]) = make_uint2(w.x, w.y);
-        *reinterpret_cast<uint2*>(&sB[buf][so1]) = make_uint2(w.z, w.w);
-        if (tid < GM_BM)
-            sdx[buf][tid] = dx;
-        else
-            sdw[buf][tid - GM_BM] = f16_bits_hw((uint16_t)dws);
-    };
-    auto compute = [&](int buf) {
-        long afr[4], bfr[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) afr[i] = *reinterpret_cast<const long*>(&sA[buf][frag_offset(wm * 64 + i * 16 + lrow, lgrp)]);
-#pragma unroll
-        for (int j = 0; j < 4; j++) bfr[j] = *reinterpret_cast<const long*>(&sB[buf][frag_offset(wn * 64 + j * 16 + lrow, lgrp)]);
-        float dwv[4];
-        f32x4 dxv[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) dwv[j] = sdw[buf][wn * 64 + j * 16 + lrow];
-#pragma unroll
-        for (int i = 0; i < 4; i++) dxv[i] = *reinterpret_cast<const f32x4*>(&sdx[buf][wm * 64 + i * 16 + lgrp * 4]);
-        const i32x4 zero = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                // C[row][col]: col = lane & 15 (weight column), row = 4*(lane>>4) + r
-                const i32x4 sv = __builtin_amdgcn_mfma_i32_16x16x32_i8(afr[i], bfr[j], zero, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    float t = (float)sv[r] * dwv[j];
-                    t = t * dxv[i][r];
-                    acc[i][j][r] = acc[i][j][r] + t;
-                }
-            }
-        }
-    };
-    uint4 a_0, a_1, a_2, a_3, w_0, w_1, w_2, w_3;
-    float dx_0, dx_1, dx_2, dx_3;
-    uint32_t dw_0, dw_1, dw_2, dw_3;
-    static_assert(GM_RS == 4, "the unrolled K loop below names four register sets");
-#define TN_GQ_SET(S) a_##S, w_##S, dx_##S, dw_##S
-#define TN_GQ_STEP(S, NEXT, B)                                    \
-    {                                                             \
-        if ((B) + GM_RS < nb) gload((B) + GM_RS, TN_GQ_SET(S));   \
-        compute((B)&1);                                           \
-        if ((B) + 1 < nb) lstore(((B) + 1) & 1, TN_GQ_SET(NEXT)); \
-        __syncthreads();                                          \
-    }
-    gload(0, TN_GQ_SET(0));
-    if (1 < nb) gload(1, TN_GQ_SET(1));
-    if (2 < nb) gload(2, TN_GQ_SET(2));
-    if (3 < nb) gload(3, TN_GQ_SET(3));
-    lstore(0, TN_GQ_SET(0));
-    __syncthreads();
-    for (int b = 0; b < nb; b += GM_RS) {
-        TN_GQ_STEP(0, 1, b)
-        if (b + 1 < nb) TN_GQ_STEP(1, 2, b + 1)
-        if (b + 2 < nb) TN_GQ_STEP(2, 3, b + 2)
-        if (b + 3 < nb) TN_GQ_STEP(3, 0, b + 3)
-    }
-#undef TN_GQ_STEP
-#undef TN_GQ_SET
-
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + wn * 64 + j * 16 + lrow;
-            if (n >= N) continue;
-            const float bv = bias ? bias[n] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm * 64 + i * 16 + lgrp * 4 + r;
-                if (m >= M) continue;
-                float v = acc[i][j][r];
-                if (bias) v = v + bv;
-                if (y_bf16)
-                    reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = bf16_from_f32(v);
-                else
-                    reinterpret_cast<float*>(y)[(int64_t)m * N + n] = v;
-            }
-        }
-    }
-}
-
 tn_status check_weight(const char* op, const char* fmt, int64_t n, int64_t k) {
     if (n < 0 || k <= 0 || k % QK != 0) {
         char buf[384];
@@ -1490,36 +850,15 @@ tn_status launch_gemv(hipStream_t st, const XT* x, int K, const uint8_t* qs, con
     return TN_OK;
 }
 
-// The q4 GEMM over the prepass's codes: 112-column tiles when they fill the
-// device in whole rounds of two workgroups per CU and 128-column ones would
-// not; when 128-column tiles would give fewer than 128 workgroups, 32-column
-// ones if they give a workgroup per CU, else 16-column ones (64 columns
-// would give fewer than 256 workgroups whenever 128 give fewer than 128).
-void gemm_q4_launch(hipStream_t st, const uint16_t* xc, const float* dxT, const float* corrT, int64_t m,
-                    int64_t M_pad, int nb, const uint8_t* qs, const uint16_t* d, int64_t n, const float* bias, void* y,
-                    int y_bf16, const float* resid) {
-    const int64_t mt = M_pad / GM_BM;
-    const bool t112 = n % 112 == 0 && (mt * (n / 112)) % 512 == 0 && (mt * cdiv(n, GM_BN)) % 512 != 0;
-    int bn = GM_BN;
-    if (mt * cdiv(n, GM_BN) < 128) bn = mt * cdiv(n, 32) >= 256 ? 32 : 16;
-#define TN_GEMM(WR, WC, TJ, BNN)                                                                                   \
-    hipLaunchKernelGGL((k_gemm<WR, WC, TJ>), dim3((unsigned)cdiv(n, BNN), (unsigned)mt), dim3(GM_THREADS), 0, st, \
-                       xc, dxT, corrT, (int)m, (int)M_pad, nb, qs, d, (int)n, bias, y, y_bf16, resid)
-    if (t112) TN_GEMM(4, 1, 7, 112);
-    else if (bn == 16) TN_GEMM(4, 1, 1, 16);
-    else if (bn == 32) TN_GEMM(4, 1, 2, 32);
-    else TN_GEMM(2, 2, 4, GM_BN);
-#undef TN_GEMM
-}
-
 template <int FMT, typename XT>
 tn_status linear_impl(hipStream_t st, const XT* x, int64_t m, int64_t k, const uint8_t* qs, const uint16_t* d,
                       int64_t n, const float* bias, void* y, int y_bf16) {
     if (m == 0 || n == 0) return TN_OK;
     const int nb = (int)(k / QK);
     const size_t ysz = y_bf16 ? 2 : 4;
-    // the GEMV reads x in 16-byte pieces; an unaligned x takes the GEMM path
-    if (m <= GEMV_MAX_M && nb <= GEMV_THREADS * Fmt<FMT>::GEMV_ITEMS && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    // the GEMV reads x in 16-byte pieces; an unaligned x takes the GEMM, whose
+    // direct loads in turn need the code plane aligned
+    if ((m <= GEMV_MAX_M || reinterpret_cast<uintptr_t>(qs) % 16 != 0) && nb <= GEMV_THREADS * Fmt<FMT>::GEMV_ITEMS && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         // decode: GEMV in chunks of up to 4 rows of x (a row's result does not
         // depend on the chunking: every output is the same recurrence)
         int64_t r = 0;
@@ -1538,52 +877,10 @@ tn_status linear_impl(hipStream_t st, const XT* x, int64_t m, int64_t k, const u
         }
         if (s == TN_OK) return TN_OK;
         if (s != TN_ENOTIMPL) return s;
-        // too large for the LDS-resident GEMV: fall through to the GEMM kernels,
-        // which compute the identical recurrence
+        // too large for the LDS-resident GEMV: the GEMM, which computes the
+        // identical recurrence
     }
-    const int64_t M_pad = cdiv(m, GM_BM) * GM_BM;
-    if (M_pad > INT32_MAX || n > INT32_MAX) return fail(TN_EVALUE, "torch._C._quantized_linear: shape too large");
-    const int64_t blocks = M_pad * nb;
-    const unsigned pgrid = (unsigned)cdiv(blocks, 8);   // 32 lanes per block
-    const unsigned vgrid = (unsigned)cdiv(blocks, 64);  // 4 lanes per block
-    const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
-    const dim3 grid((unsigned)cdiv(n, GM_BN), (unsigned)(M_pad / GM_BM));
-    const size_t dx_bytes = (size_t)M_pad * nb * 4;
-    void* ws = nullptr;
-    if constexpr (FMT == FMT_Q8_0) {
-        const size_t xc_bytes = (size_t)M_pad * k;
-        tn_status s = workspace(st, xc_bytes + dx_bytes, &ws);
-        if (s != TN_OK) return s;
-        int8_t* xc = static_cast<int8_t*>(ws);
-        float* dxT = reinterpret_cast<float*>(static_cast<char*>(ws) + xc_bytes);
-        if (aligned)
-            hipLaunchKernelGGL((k_q8_rows_i8_v<XT>), dim3(vgrid), dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb,
-                               xc, dxT);
-        else
-            hipLaunchKernelGGL((k_q8_rows_i8<XT>), dim3(pgrid), dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb,
-                               xc, dxT);
-        TN_LAUNCHED();
-        hipLaunchKernelGGL(k_gemm_q8, grid, dim3(GM_THREADS), 0, st, xc, dxT, (int)m, (int)M_pad, nb, qs, d, (int)n,
-                           bias, y, y_bf16);
-        TN_LAUNCHED();
-    } else {
-        const size_t xc_bytes = (size_t)M_pad * k * 2;
-        tn_status s = workspace(st, xc_bytes + 2 * dx_bytes, &ws);
-        if (s != TN_OK) return s;
-        uint16_t* xc = static_cast<uint16_t*>(ws);
-        float* dxT = reinterpret_cast<float*>(static_cast<char*>(ws) + xc_bytes);
-        float* corrT = reinterpret_cast<float*>(static_cast<char*>(ws) + xc_bytes + dx_bytes);
-        if (aligned)
-            hipLaunchKernelGGL((k_q8_rows_v<XT>), dim3(vgrid), dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb, xc,
-                               dxT, corrT);
-        else
-            hipLaunchKernelGGL((k_q8_rows<XT>), dim3(pgrid), dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb, xc,
-                               dxT, corrT);
-        TN_LAUNCHED();
-        gemm_q4_launch(st, xc, dxT, corrT, m, M_pad, nb, qs, d, n, bias, y, y_bf16, nullptr);
-        TN_LAUNCHED();
-    }
-    return TN_OK;
+    return qgemm_launch(st, QGemmArgs{FMT, x, sizeof(XT) == 2, m, k, XM_ROWS, 0, qs, d, n, bias, y, y_bf16, nullptr});
 }
 
 // The codec entry points of one format.
@@ -1703,32 +1000,7 @@ tn_status linear_prefill(hipStream_t st, const float* x, int64_t m, int64_t k, i
     if (reinterpret_cast<uintptr_t>(x) % 16 != 0) return fail(TN_EINVAL, "linear_prefill: x must be 16-byte aligned");
     if (xm == XM_HEADS && (hd <= 0 || hd % QK != 0 || k % hd != 0))
         return fail(TN_EINVAL, "linear_prefill: the head dim must divide the row and be a multiple of 32");
-    const int nb = (int)(k / QK);
-    const int64_t M_pad = cdiv(m, GM_BM) * GM_BM;
-    if (M_pad > INT32_MAX || n > INT32_MAX || M_pad * k * (xm == XM_GLU ? 2 : 1) > INT32_MAX)
-        return fail(TN_EVALUE, "linear_prefill: shape too large");
-    const int64_t blocks = M_pad * nb;
-    const size_t dx_bytes = (size_t)M_pad * nb * 4, xc_bytes = (size_t)M_pad * k * 2;
-    void* ws = nullptr;
-    s = workspace(st, xc_bytes + 2 * dx_bytes, &ws);
-    if (s != TN_OK) return s;
-    uint16_t* xc = static_cast<uint16_t*>(ws);
-    float* dxT = reinterpret_cast<float*>(static_cast<char*>(ws) + xc_bytes);
-    float* corrT = reinterpret_cast<float*>(static_cast<char*>(ws) + xc_bytes + dx_bytes);
-    const dim3 vgrid((unsigned)cdiv(blocks, 64));  // 4 lanes per block
-    if (xm == XM_GLU)
-        hipLaunchKernelGGL((k_q8_rows_v<float, XM_GLU>), vgrid, dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb, xc,
-                           dxT, corrT, 0);
-    else if (xm == XM_HEADS)
-        hipLaunchKernelGGL((k_q8_rows_v<float, XM_HEADS>), vgrid, dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb,
-                           xc, dxT, corrT, hd);
-    else
-        hipLaunchKernelGGL((k_q8_rows_v<float, XM_ROWS>), vgrid, dim3(256), 0, st, x, (int)m, (int)M_pad, (int)k, nb,
-                           xc, dxT, corrT, 0);
-    TN_LAUNCHED();
-    gemm_q4_launch(st, xc, dxT, corrT, m, M_pad, nb, qs, d, n, nullptr, y, 0, resid);
-    TN_LAUNCHED();
-    return TN_OK;
+    return qgemm_launch(st, QGemmArgs{FMT_Q4_0, x, 0, m, k, xm, hd, qs, d, n, nullptr, y, 0, resid});
 }
 
 }  // namespace tn
