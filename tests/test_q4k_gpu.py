@@ -181,3 +181,21 @@ def test_batched_rows_equal_one_row_calls_and_bf16_io(tn):
     yb = tn._quantized_linear(xb, q, out_dtype="bfloat16").bits()
     want = O.q4_k_linear(xb.numpy(), tn._quantized_blob(q), n, threads=8)
     assert np.array_equal(yb, O.bf16_from_f32(want))
+
+
+def test_writer_on_rows_off_the_usual_path(tn):
+    """The writer keeps a step's scale and offset instead of its levels: rows
+    where it falls back on the search's levels (a zero d), and values whose
+    scaled elements leave the range of the level rounding, byte for byte."""
+    rng = np.random.default_rng(77)
+    rows = [rng.standard_normal(256) * s for s in (1e-30, 1e-20, 1e-8, 1e-4, 1.0, 1e4, 6e4, 1e10, 1e20)]
+    rows.append(np.repeat(rng.standard_normal(8), 32))  # constant sub-blocks
+    rows.append(np.where(np.arange(256) < 32, 1e4, 1e-4) * rng.standard_normal(256))  # sub-blocks whose scale rounds to 0
+    rows.append(np.where(np.arange(256) % 32 == 0, 3e38, 1.0) * rng.standard_normal(256))  # errors overflow
+    rows.append(np.abs(rng.standard_normal(256)) + 5.0)  # no negative value
+    rows.append(-np.abs(rng.standard_normal(256)) - 5.0)
+    rows.append(np.round(rng.standard_normal(256) * 3))  # ties
+    x = np.stack(rows).astype(np.float32)
+    got = tn._quantized_blob(tn._quantize(tn.tensor(x, device="hip"), "q4_k"))
+    want = O.q4_k_quantize(x)
+    assert bytes(got) == bytes(want), [i for i in range(len(rows)) if got[144 * i:144 * i + 144] != want[144 * i:144 * i + 144]]

@@ -128,12 +128,33 @@ __global__ void k_qk_dequantize(const uint8_t* __restrict__ w, int64_t nsb, floa
 // reference's operation order; the super-block's max scale and max min are
 // taken in sub-block order, as the reference's loop does.
 
-__device__ float make_qkx2(const float* x, const float* w, uint8_t* L, float* the_min) {
+// What bounds it: VALU. 18 instructions per element and step, each rounding
+// the reference's (two for the scaled element, four for its level, six for the
+// three sums, six for the error), 21 steps: 12,000 per lane, all in registers.
+// The levels of the best step are not stored: the step's scale and offset give
+// them again, and only a sub-block whose final d is zero needs them. [4096, 4096]
+// took 1410 us with the levels in byte arrays, 156 us so (three waves per SIMD).
+
+// The level of t as a float, clamped to 0 .. 15: nearest_int_even and the clamp
+// as integers on the biased sum's bits (every t, out of range and NaN included,
+// gives what the reference's masked bits give), then the bias taken off.
+__device__ inline float level_of(float t) {
+    constexpr uint32_t BIAS = 0x4b400000u;  // 12582912.0f
+    const uint32_t b = (__float_as_uint(t + 12582912.0f) & 0x007fffffu) | 0x4b000000u;
+    const int c = min(max((int)b, (int)BIAS), (int)(BIAS + 15u));
+    return __int_as_float(c) - 12582912.0f;
+}
+
+// Returns the scale; *the_min, and the (iscale, offset) whose levels
+// level_of(iscale * (x - offset)) the search chose (iscale 0: all levels 0).
+__device__ __attribute__((always_inline)) inline float make_qkx2(const float (&x)[32], const float (&w)[32], float* the_min,
+                                                                 float* lscale, float* loff) {
     constexpr int n = 32, nmax = 15, nstep = 20;
     const float rmin = -1.0f, rdelta = 0.1f;
     float mn = x[0], mx = x[0];
     float sum_w = w[0];
     float sum_x = sum_w * x[0];
+#pragma unroll
     for (int i = 1; i < n; i++) {
         if (x[i] < mn) mn = x[i];
         if (x[i] > mx) mx = x[i];
@@ -142,33 +163,34 @@ __device__ float make_qkx2(const float* x, const float* w, uint8_t* L, float* th
     }
     if (mn > 0.0f) mn = 0.0f;
     if (mx == mn) {
-        for (int i = 0; i < n; i++) L[i] = 0;
+        *lscale = 0.0f;
+        *loff = 0.0f;
         *the_min = -mn;
         return 0.0f;
     }
     float iscale = (float)nmax / (mx - mn);
     float scale = 1.0f / iscale;
     float best = 0.0f;
+    *lscale = iscale;
+    *loff = mn;
+#pragma unroll
     for (int i = 0; i < n; i++) {
-        int li = nearest_int_even(iscale * (x[i] - mn));
-        li = li < 0 ? 0 : (li > nmax ? nmax : li);
-        L[i] = (uint8_t)li;
-        float diff = scale * (float)li + mn - x[i];
+        float diff = scale * level_of(iscale * (x[i] - mn)) + mn - x[i];
         diff = diff * diff;
         best = best + w[i] * diff;
     }
-    uint8_t laux[32];
+#pragma unroll 1
     for (int is = 0; is <= nstep; is++) {
         iscale = (rmin + rdelta * (float)is + (float)nmax) / (mx - mn);
         float sum_l = 0.0f, sum_l2 = 0.0f, sum_xl = 0.0f;
+        float lf[n];
+#pragma unroll
         for (int i = 0; i < n; i++) {
-            int li = nearest_int_even(iscale * (x[i] - mn));
-            li = li < 0 ? 0 : (li > nmax ? nmax : li);
-            laux[i] = (uint8_t)li;
-            const float lf = (float)li;
-            sum_l = sum_l + w[i] * lf;
-            sum_l2 = sum_l2 + w[i] * lf * lf;
-            sum_xl = sum_xl + w[i] * lf * x[i];
+            lf[i] = level_of(iscale * (x[i] - mn));
+            const float wl = w[i] * lf[i];
+            sum_l = sum_l + wl;
+            sum_l2 = sum_l2 + wl * lf[i];
+            sum_xl = sum_xl + wl * x[i];
         }
         const float D = sum_w * sum_l2 - sum_l * sum_l;
         if (D > 0.0f) {
@@ -179,13 +201,15 @@ __device__ float make_qkx2(const float* x, const float* w, uint8_t* L, float* th
                 this_scale = sum_xl / sum_l2;
             }
             float cur = 0.0f;
+#pragma unroll
             for (int i = 0; i < n; i++) {
-                float diff = this_scale * (float)laux[i] + this_min - x[i];
+                float diff = this_scale * lf[i] + this_min - x[i];
                 diff = diff * diff;
                 cur = cur + w[i] * diff;
             }
             if (cur < best) {
-                for (int i = 0; i < n; i++) L[i] = laux[i];
+                *lscale = iscale;
+                *loff = mn;
                 best = cur;
                 scale = this_scale;
                 mn = this_min;
@@ -203,8 +227,9 @@ __global__ __launch_bounds__(256) void k_qk_quantize(const float* __restrict__ x
     const int64_t sb = t >> 3;
     const bool live = sb < nsb;  // the 8 lanes of a super-block are live together
     float x[32], w[32];
-    uint8_t L[32];
-    float scale = 0.0f, mnv = 0.0f;
+    float scale = 0.0f, mnv = 0.0f, lscale = 0.0f, loff = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; i++) x[i] = 0.0f;
     if (live) {
         const float4* src = reinterpret_cast<const float4*>(xin + sb * QKK + 32 * j);
 #pragma unroll
@@ -213,10 +238,12 @@ __global__ __launch_bounds__(256) void k_qk_quantize(const float* __restrict__ x
             x[4 * i] = v.x; x[4 * i + 1] = v.y; x[4 * i + 2] = v.z; x[4 * i + 3] = v.w;
         }
         float sum_x2 = 0.0f;
+#pragma unroll
         for (int i = 0; i < 32; i++) sum_x2 = sum_x2 + x[i] * x[i];
         const float av_x = sqrtf(sum_x2 / 32.0f);
+#pragma unroll
         for (int i = 0; i < 32; i++) w[i] = av_x + fabsf(x[i]);
-        scale = make_qkx2(x, w, L, &mnv);
+        scale = make_qkx2(x, w, &mnv, &lscale, &loff);
     }
     // max scale and max min over the super-block, in sub-block order, from +0
     const int lane = (int)(threadIdx.x & 63), base = lane & ~7;
@@ -238,12 +265,13 @@ __global__ __launch_bounds__(256) void k_qk_quantize(const float* __restrict__ x
     const uint16_t mh = f16_from_f32(max_min / 63.0f);
     // the final levels; a sub-block whose d is zero keeps the search's levels
     const float d = f16_to_f32(dh) * (float)ls;
-    if (live && d != 0.0f) {
-        const float dm = f16_to_f32(mh) * (float)lm;
-        for (int i = 0; i < 32; i++) {
-            int lv = nearest_int_even((x[i] + dm) / d);
-            L[i] = (uint8_t)(lv < 0 ? 0 : (lv > 15 ? 15 : lv));
-        }
+    const float dm = f16_to_f32(mh) * (float)lm;
+    uint32_t L[32];
+#pragma unroll
+    for (int i = 0; i < 32; i++) {
+        // the search's levels where d is zero: 0 if it chose none
+        const float t = d != 0.0f ? (x[i] + dm) / d : lscale * (x[i] - loff);
+        L[i] = d == 0.0f && lscale == 0.0f ? 0u : (uint32_t)level_of(t);
     }
     // the packed 6-bit scales (k_quants.rs:1625-1635) from all eight lanes
     int lsv[8], lmv[8];
@@ -257,7 +285,7 @@ __global__ __launch_bounds__(256) void k_qk_quantize(const float* __restrict__ x
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         // position-major: dword l holds elements l, 8 + l, 16 + l, 24 + l
-        mine[q] = (uint32_t)L[q] | ((uint32_t)L[8 + q] << 8) | ((uint32_t)L[16 + q] << 16) | ((uint32_t)L[24 + q] << 24);
+        mine[q] = L[q] | (L[8 + q] << 8) | (L[16 + q] << 16) | (L[24 + q] << 24);
     }
 #pragma unroll
     for (int q = 0; q < 8; q++) other[q] = __shfl((int)mine[q], lane ^ 1, 64);
