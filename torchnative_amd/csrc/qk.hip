@@ -340,6 +340,10 @@ __global__ __launch_bounds__(256) void k_qk_quantize(const float* __restrict__ x
 
 constexpr int QG_THREADS = 256;
 constexpr int QG_TERMS = 9;
+// LDS strides of a super-block's codes and code sums: 16 bytes over 256 and 64
+// (`pad`), so that the lanes of a wave, each at its own super-block, read
+// different banks (without it every 16-byte read of eight lanes met one bank
+// eight times). Rows so long that only the unpadded layout fits run unpadded.
 
 template <typename XT>
 __device__ inline float4 load4(const XT* p);
@@ -352,61 +356,58 @@ __device__ inline float4 load4<uint16_t>(const uint16_t* p) {
                        bf16_to_f32((uint16_t)(h.y & 0xffffu)), bf16_to_f32((uint16_t)(h.y >> 16)));
 }
 
+// Q8_K of one super-block held four elements a lane (BlockQ8K::from_float,
+// k_quants.rs:2375-2413): the first element of the largest |x| (a NaN is never
+// taken) gives iscale = -127 / it; codes to q, the sum of this lane's four
+// lanes' codes (16 elements) to *sum, d = 1 / iscale or 0 is returned. The
+// largest is a DPP reduction, the first lane that holds it a ballot.
+__device__ __attribute__((always_inline)) inline float q8k_wave(const float4& v4, int (&q)[4], int* sum) {
+    const float e[4] = {v4.x, v4.y, v4.z, v4.w};
+    float am = 0.0f, mv = 0.0f;  // this lane's first largest (strict <)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (am < fabsf(e[i])) { am = fabsf(e[i]); mv = e[i]; }
+    const float top = xor32_max(xor16_max(row16_max(am)));
+    float d = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = 0;
+    if (top != 0.0f) {  // uniform
+        const int first = __ffsll((unsigned long long)__ballot(am == top)) - 1;
+        const float iscale = -127.0f / __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mv), first));
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = sat_i8k(roundf(iscale * e[i]));
+        d = 1.0f / iscale;
+    }
+    int s = q[0] + q[1] + q[2] + q[3];
+    s = s + dpp_i<0xB1>(s);
+    *sum = s + dpp_i<0x4E>(s);
+    return d;
+}
+
 template <int MR, typename XT>
 __global__ __launch_bounds__(QG_THREADS) void k_gemv_qk(const XT* __restrict__ x, int K, int nsb,
-                                                       const uint8_t* __restrict__ w, int N, int rows,
+                                                       const uint8_t* __restrict__ w, int N, int rows, int pad,
                                                        const float* __restrict__ bias, void* y, int y_bf16) {
+    const int xs = QKK + 16 * pad, bs = 16 + 4 * pad;
     extern __shared__ __align__(16) char smem[];
-    int8_t* xq = reinterpret_cast<int8_t*>(smem);                     // [MR][nsb][256] position-major
-    float* xd = reinterpret_cast<float*>(smem + (size_t)MR * K);      // [MR][nsb], padded to 16 bytes
-    int* xbs = reinterpret_cast<int*>(xd + ((MR * nsb + 3) & ~3));    // [MR][nsb][16]
-    float* terms = reinterpret_cast<float*>(xbs + MR * nsb * 16);      // [2][rows*MR][nsb][9]
+    int8_t* xq = reinterpret_cast<int8_t*>(smem);                               // [MR][nsb][xs] position-major
+    float* xd = reinterpret_cast<float*>(smem + (size_t)MR * nsb * xs);      // [MR][nsb], padded to 16 bytes
+    int* xbs = reinterpret_cast<int*>(xd + ((MR * nsb + 3) & ~3));              // [MR][nsb][bs]
+    float* terms = reinterpret_cast<float*>(xbs + MR * nsb * bs);             // [2][rows*MR][nsb][9]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int ntiles = (N + rows - 1) / rows;
 
-    // phase 1: Q8_K of the activation rows (BlockQ8K::from_float)
-    for (int blk = wave; blk < MR * nsb; blk += QG_THREADS / 64) {
-        const int mr = blk / nsb, sb = blk - mr * nsb;
-        const float4 v4 = load4<XT>(x + (int64_t)mr * K + sb * QKK + 4 * lane);
-        const float e[4] = {v4.x, v4.y, v4.z, v4.w};
-        // this lane's first largest |x| (strict <, NaN never taken), then the
-        // wave's: larger value wins, equal values go to the lower index
-        float am = 0.0f, mv = 0.0f;
-        int idx = 0x7fffffff;
+    // The first activation blocks of each wave are requested before the first
+    // tile's weights, which are then in flight during phase 1.
+    constexpr int HOLD = 4;
+    float4 xv[HOLD];
+    const int nblk = MR * nsb;
+    auto xload = [&](int blk) {
+        const int b = min(blk, nblk - 1), mr = b / nsb;
+        return load4<XT>(x + (int64_t)mr * K + (b - mr * nsb) * QKK + 4 * lane);
+    };
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            if (am < fabsf(e[i])) { am = fabsf(e[i]); mv = e[i]; idx = 4 * lane + i; }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            const float oa = __shfl_xor(am, off, 64), ov = __shfl_xor(mv, off, 64);
-            const int oi = __shfl_xor(idx, off, 64);
-            if (oa > am || (oa == am && oi < idx)) { am = oa; mv = ov; idx = oi; }
-        }
-        int q[4] = {0, 0, 0, 0};
-        float d = 0.0f;
-        if (am != 0.0f) {
-            const float iscale = -127.0f / mv;
-#pragma unroll
-            for (int i = 0; i < 4; i++) q[i] = sat_i8k(roundf(iscale * e[i]));
-            d = 1.0f / iscale;
-        }
-        // element e = 4*lane + i: sub-block j = lane / 8, within it r = 4*(lane % 8) + i,
-        // g = r / 8, l = r % 8 -> position-major byte 32 j + 4 l + g
-        int8_t* dst = xq + (int64_t)blk * QKK;
-        const int j = lane >> 3, r0 = 4 * (lane & 7);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int r = r0 + i;
-            dst[32 * j + 4 * (r & 7) + (r >> 3)] = (int8_t)q[i];
-        }
-        // sums of 16 codes: lanes 4s .. 4s + 3 hold elements 16s .. 16s + 15
-        int s = q[0] + q[1] + q[2] + q[3];
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        if ((lane & 3) == 0) xbs[blk * 16 + (lane >> 2)] = (int)(int16_t)s;
-        if (lane == 0) xd[blk] = d;
-    }
-    __syncthreads();
+    for (int u = 0; u < HOLD; u++) xv[u] = xload(wave + u * (QG_THREADS / 64));
 
     // phases 2 and 3, persistent over row tiles with the next tile's bytes in flight
     // The super-block loads are unconditional buffer loads over the tile's
@@ -430,6 +431,30 @@ __global__ __launch_bounds__(QG_THREADS) void k_gemv_qk(const XT* __restrict__ x
     };
     int tile = (int)blockIdx.x;
     gload(tile, wv);  // the grid never exceeds the tile count
+    __builtin_amdgcn_sched_barrier(0);
+
+    // phase 1: Q8_K of the activation rows
+    auto quantise = [&](const float4& v4, int blk) __attribute__((always_inline)) {
+        int q[4], s;
+        const float d = q8k_wave(v4, q, &s);
+        // element e = 4*lane + i: sub-block j = lane / 8, within it r = 4*(lane % 8) + i,
+        // g = r / 8, l = r % 8 -> position-major byte 32 j + 4 l + g
+        int8_t* dst = xq + blk * xs;
+        const int j = lane >> 3, r0 = 4 * (lane & 7);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = r0 + i;
+            dst[32 * j + 4 * (r & 7) + (r >> 3)] = (int8_t)q[i];
+        }
+        if ((lane & 3) == 0) xbs[blk * bs + (lane >> 2)] = (int)(int16_t)s;
+        if (lane == 0) xd[blk] = d;
+    };
+#pragma unroll
+    for (int u = 0; u < HOLD; u++)
+        if (wave + u * (QG_THREADS / 64) < nblk) quantise(xv[u], wave + u * (QG_THREADS / 64));
+    for (int blk = wave + HOLD * (QG_THREADS / 64); blk < nblk; blk += QG_THREADS / 64) quantise(xload(blk), blk);
+    __syncthreads();
+
     for (int buf = 0; tile < ntiles; tile += (int)gridDim.x, buf ^= 1) {
         gload(tile + (int)gridDim.x, wn);
         const int64_t row0 = (int64_t)tile * rows;
@@ -449,7 +474,7 @@ __global__ __launch_bounds__(QG_THREADS) void k_gemv_qk(const XT* __restrict__ x
 #pragma unroll
             for (int mr = 0; mr < MR; mr++) {
                 const int blk = mr * nsb + sb;
-                const int* xa = reinterpret_cast<const int*>(xq + (int64_t)blk * QKK);
+                const int* xa = reinterpret_cast<const int*>(xq + blk * xs);
                 int aux[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
@@ -464,15 +489,16 @@ __global__ __launch_bounds__(QG_THREADS) void k_gemv_qk(const XT* __restrict__ x
                     for (int l = 0; l < 8; l++) {
                         const int lo = __builtin_amdgcn_sdot4((int)(dws[l] & 0x0f0f0f0fu), xs[l], 0, false);
                         const int hi = __builtin_amdgcn_sdot4((int)((dws[l] >> 4) & 0x0f0f0f0fu), xs[8 + l], 0, false);
-                        aux[l] += sc[2 * c] * lo + sc[2 * c + 1] * hi;
+                        // |lo|, |hi| <= 4 * 15 * 127: 24-bit products (full rate, a 32-bit one takes four times as long)
+                        aux[l] += __mul24(sc[2 * c], lo) + __mul24(sc[2 * c + 1], hi);
                     }
                 }
-                const int4* bs4 = reinterpret_cast<const int4*>(xbs + blk * 16);
+                const int4* bs4 = reinterpret_cast<const int4*>(xbs + blk * bs);
                 int sumi = 0;
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
                     const int4 bs = bs4[u];
-                    sumi += bs.x * mn[2 * u] + bs.y * mn[2 * u] + bs.z * mn[2 * u + 1] + bs.w * mn[2 * u + 1];
+                    sumi += __mul24(bs.x + bs.y, mn[2 * u]) + __mul24(bs.z + bs.w, mn[2 * u + 1]);
                 }
                 const float yd = xd[blk];
                 const float d = dw * yd;
@@ -565,30 +591,10 @@ __global__ __launch_bounds__(256) void k_q8k_rows(const XT* __restrict__ x, int 
     const int lane = threadIdx.x & 63;
     if (blk >= (int64_t)M_pad * nsb) return;
     const int row = (int)(blk / nsb), sb = (int)(blk - (int64_t)row * nsb);
-    float e[4] = {0.f, 0.f, 0.f, 0.f};
-    if (row < M) {
-        const float4 v4 = load4<XT>(x + (int64_t)row * K + sb * QKK + 4 * lane);
-        e[0] = v4.x; e[1] = v4.y; e[2] = v4.z; e[3] = v4.w;
-    }
-    float am = 0.0f, mv = 0.0f;
-    int idx = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (am < fabsf(e[i])) { am = fabsf(e[i]); mv = e[i]; idx = 4 * lane + i; }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float oa = __shfl_xor(am, off, 64), ov = __shfl_xor(mv, off, 64);
-        const int oi = __shfl_xor(idx, off, 64);
-        if (oa > am || (oa == am && oi < idx)) { am = oa; mv = ov; idx = oi; }
-    }
-    int q[4] = {0, 0, 0, 0};
-    float d = 0.0f;
-    if (am != 0.0f) {
-        const float iscale = -127.0f / mv;
-#pragma unroll
-        for (int i = 0; i < 4; i++) q[i] = sat_i8k(roundf(iscale * e[i]));
-        d = 1.0f / iscale;
-    }
+    float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row < M) v4 = load4<XT>(x + (int64_t)row * K + sb * QKK + 4 * lane);
+    int q[4], s;
+    const float d = q8k_wave(v4, q, &s);
     uint16_t* dst = xa + blk * QKK;
     const int j = lane >> 3, G = j >> 1, h = j & 1;
 #pragma unroll
@@ -596,9 +602,6 @@ __global__ __launch_bounds__(256) void k_q8k_rows(const XT* __restrict__ x, int 
         const int r = 4 * (lane & 7) + i, g = r >> 3, l = r & 7;
         dst[(l * 4 + G) * 8 + 4 * h + gslot(g)] = __builtin_bit_cast(uint16_t, (_Float16)(float)q[i]);
     }
-    int s = q[0] + q[1] + q[2] + q[3];
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
     if ((lane & 3) == 0) xbs[blk * 16 + (lane >> 2)] = __builtin_bit_cast(uint16_t, (_Float16)(float)s);
     if (lane == 0) xd[(int64_t)sb * M_pad + row] = d;
 }
@@ -783,9 +786,9 @@ tn_status check_qk(const char* op, int64_t n, int64_t k) {
     return TN_OK;
 }
 
-size_t qk_lds(int mr, int k, int rows) {
-    const int nsb = k / QKK;
-    return (size_t)mr * k + (size_t)((mr * nsb + 3) & ~3) * 4 + (size_t)mr * nsb * 64 +
+size_t qk_lds(int mr, int k, int rows, int pad) {
+    const int nsb = k / QKK, xs = QKK + 16 * pad, bs = 16 + 4 * pad;
+    return (size_t)mr * nsb * xs + (size_t)((mr * nsb + 3) & ~3) * 4 + (size_t)mr * nsb * bs * 4 +
            2 * (size_t)rows * mr * nsb * QG_TERMS * 4;
 }
 
@@ -798,15 +801,17 @@ tn_status launch_gemv_qk(hipStream_t st, const XT* x, int K, const uint8_t* w, i
     if (rows > spread) rows = spread;
     if (rows > N) rows = N;
     if (rows < 1) return TN_ENOTIMPL;
-    const size_t lds = qk_lds(MR, K, rows);
+    int pad = 1;
+    size_t lds = qk_lds(MR, K, rows, pad);
+    if (lds > 64 * 1024) lds = qk_lds(MR, K, rows, pad = 0);
     if (lds > 64 * 1024) return TN_ENOTIMPL;
     int resident = 0;
     tn_status s = resident_workgroups(reinterpret_cast<const void*>(&k_gemv_qk<MR, XT>), QG_THREADS, lds, &resident);
     if (s != TN_OK) return s;
     const int64_t ntiles = cdiv(N, rows);
     const unsigned grid = (unsigned)(ntiles < resident ? ntiles : resident);
-    hipLaunchKernelGGL((k_gemv_qk<MR, XT>), dim3(grid), dim3(QG_THREADS), lds, st, x, K, nsb, w, N, rows, bias, y,
-                       y_bf16);
+    hipLaunchKernelGGL((k_gemv_qk<MR, XT>), dim3(grid), dim3(QG_THREADS), lds, st, x, K, nsb, w, N, rows, pad, bias,
+                       y, y_bf16);
     TN_LAUNCHED();
     return TN_OK;
 }
