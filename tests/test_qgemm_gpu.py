@@ -108,3 +108,39 @@ def test_operands_at_any_element(tn, fmt):
     _lib.check(fn(None, x.data_ptr(), _lib.TN_F32, m, k, moved.data_ptr() + 8, q._d.data_ptr(), n, None, y.data_ptr(),
                   _lib.TN_F32))
     assert y.numpy().tobytes() == _linear(fmt)(x.numpy(), blob, n, threads=8).tobytes()
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+def test_large_products_of_two_to_four_rows(tn, fmt):
+    """m n past the line where they leave the GEMV: the oracle's bits, and the
+    same bits from a captured call on a stream without a workspace, which
+    stays on the GEMV (three replays)."""
+    import ctypes
+
+    from torchnative_amd import _lib as L
+
+    f = L.lib()
+    k, n = 1024, 20000
+    blob = _blob(fmt, n, k, 9)
+    q = tn._quantized_from_blob(blob, (n, k), fmt, device="hip")
+    for m in (2, 3, 4):
+        x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+        xd, y = tn.tensor(x, device="hip"), tn.empty((m, n), "float32", "hip")
+        want = _linear(fmt)(x, blob, n, threads=16)
+        assert tn._quantized_linear(xd, q).numpy().tobytes() == want.tobytes()
+        s, g = ctypes.c_void_p(), ctypes.c_void_p()
+        L.check(f.tn_stream_create(ctypes.byref(s)))
+        try:
+            L.check(f.tn_stream_begin_capture(s))
+            L.check(getattr(f, f"tn_{fmt}_linear")(s, xd.data_ptr(), L.TN_F32, m, k, *q._planes(), n, None, y.data_ptr(),
+                                                   L.TN_F32))
+            L.check(f.tn_stream_end_capture(s, ctypes.byref(g)))
+            for _ in range(3):
+                y.zero_()
+                tn.synchronize()
+                L.check(f.tn_graph_launch(s, g))
+                L.check(f.tn_stream_synchronize(s))
+                assert y.numpy().tobytes() == want.tobytes()
+            L.check(f.tn_graph_destroy(g))
+        finally:
+            L.check(f.tn_stream_destroy(s))

@@ -20,6 +20,8 @@ struct QGemmArgs {
     const float* resid;  // added after the sum (and bias), may be y
 };
 
+// Bytes of the stream's workspace that qgemm_launch uses.
+inline size_t qgemm_workspace(const QGemmArgs& a) { return (size_t)(cdiv(a.m, 16) * 16 * (a.k / QK)) * (32 + 4); }
 // Quantises the rows into the stream's workspace, then the product.
 tn_status qgemm_launch(hipStream_t st, const QGemmArgs& a);
 

@@ -362,7 +362,7 @@ tn_status qgemm_launch(hipStream_t st, const QGemmArgs& a) {
         return fail(TN_EVALUE, "torch._C._quantized_linear: shape too large");
     void* ws = nullptr;
     const size_t xbytes = (size_t)blocks * 32;
-    TN_TRY(workspace(st, xbytes + (size_t)blocks * 4, &ws));
+    TN_TRY(workspace(st, qgemm_workspace(a), &ws));
     uint8_t* xf = static_cast<uint8_t*>(ws);
     float* dxf = reinterpret_cast<float*>(xf + xbytes);
     const float unit = a.fmt == FMT_Q4_0 ? 0.0625f : 1.0f;

@@ -856,6 +856,20 @@ tn_status linear_impl(hipStream_t st, const XT* x, int64_t m, int64_t k, const u
     if (m == 0 || n == 0) return TN_OK;
     const int nb = (int)(k / QK);
     const size_t ysz = y_bf16 ? 2 : 4;
+    const QGemmArgs rows{FMT, x, sizeof(XT) == 2, m, k, XM_ROWS, 0, qs, d, n, bias, y, y_bf16, nullptr};
+    // Two to four rows: the GEMV's time grows with the work (0.13 us per
+    // million of m n k beyond its launch), the GEMM's with k alone (about 7 us +
+    // 2.7 us per 1024 of k up to n = 16384), so a large product goes there: [4, 4096]
+    // x [14336, 4096] 33.9 -> 17.8 us, three rows 25.2 -> 18.0, two 19.8 -> 17.5,
+    // [4, 1024] x [16000, 1024] 9.9 -> 8.6. Short rows stay ([3, 576] x [49152, 576]:
+    // 8.7, and 10.4 there). It needs the stream's workspace; a capture that could
+    // not grow it keeps the GEMV.
+    if (m >= 2 && m <= GEMV_MAX_M && k >= 1024 && m * n > 16384 + 44000000 / k &&
+        reinterpret_cast<uintptr_t>(qs) % 16 == 0) {
+        void* ws = nullptr;
+        TN_TRY(workspace_or_none(st, qgemm_workspace(rows), &ws));
+        if (ws) return qgemm_launch(st, rows);
+    }
     // the GEMV reads x in 16-byte pieces; an unaligned x takes the GEMM, whose
     // direct loads in turn need the code plane aligned
     if ((m <= GEMV_MAX_M || reinterpret_cast<uintptr_t>(qs) % 16 != 0) && nb <= GEMV_THREADS * Fmt<FMT>::GEMV_ITEMS && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
@@ -880,7 +894,7 @@ tn_status linear_impl(hipStream_t st, const XT* x, int64_t m, int64_t k, const u
         // too large for the LDS-resident GEMV: the GEMM, which computes the
         // identical recurrence
     }
-    return qgemm_launch(st, QGemmArgs{FMT, x, sizeof(XT) == 2, m, k, XM_ROWS, 0, qs, d, n, bias, y, y_bf16, nullptr});
+    return qgemm_launch(st, rows);
 }
 
 // The codec entry points of one format.
