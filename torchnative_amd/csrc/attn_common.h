@@ -170,6 +170,87 @@ __device__ __attribute__((always_inline)) inline f32x4 mask_quad(const MaskRef m
 
 
 
+// A mask's quads (keys key .. key+3 of one row, key a multiple of four) requested
+// in one place and read in another, so that their latency passes under other
+// work. For masks with dense keys whose (batch, head) plane a descriptor reaches
+// (mask_ahead). A quad is read as the aligned dwords that hold it: up to three
+// bytes of the dwords at either end of the plane lie outside of it, in the same
+// aligned dword as bytes inside. What stands for keys at or past S is undefined.
+struct MaskRow {
+    buf_rsrc r;
+    uint32_t off;    // the row's aligned byte offset
+    uint32_t shift;  // bits of the first dword before the quad
+    // row qi of plane (b, h), elements of es bytes
+    __device__ __attribute__((always_inline)) inline MaskRow(const MaskRef& m, int es, int b, int h, int qi, int L,
+                                                             int S)
+        : r(desc(m, es, b, h, L, S)) {
+        const uint32_t o = (uint32_t)(reinterpret_cast<uintptr_t>(plane(m, es, b, h)) & 3) +
+                           (uint32_t)qi * (uint32_t)m.sl * (uint32_t)es;
+        off = qi < L ? o & ~3u : BUF_OOB;
+        shift = 8 * (o & 3);
+    }
+    __device__ static inline const char* plane(const MaskRef& m, int es, int b, int h) {
+        return static_cast<const char*>(m.p) + ((int64_t)b * m.sb + (int64_t)h * m.sh) * es;
+    }
+    __device__ static inline buf_rsrc desc(const MaskRef& m, int es, int b, int h, int L, int S) {
+        const char* p = plane(m, es, b, h);
+        const uintptr_t lead = reinterpret_cast<uintptr_t>(p) & 3;
+        return make_rsrc(p - lead, ((uint32_t)lead + (uint32_t)(((int64_t)(L - 1) * m.sl + S) * es) + 3) & ~3u);
+    }
+};
+
+// dwords that hold a quad in format MASK
+template <int MASK>
+constexpr int MASK_W = MASK == 1 ? 4 : MASK == 3 ? 2 : 3;
+
+// the additive values, natural units, of a quad whose dwords are v
+template <int MASK, bool F16, class V>
+__device__ __attribute__((always_inline)) inline f32x4 mask_values(V v, uint32_t shift) {
+    if constexpr (MASK == 1) {
+        return (f32x4){__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]), __uint_as_float(v[3])};
+    } else if constexpr (MASK == 3) {
+        const uint32_t w = __builtin_amdgcn_alignbit(v[1], v[0], shift);
+        return (f32x4){(w & 0xffu) ? 0.0f : -INFINITY, (w & 0xff00u) ? 0.0f : -INFINITY,
+                       (w & 0xff0000u) ? 0.0f : -INFINITY, (w & 0xff000000u) ? 0.0f : -INFINITY};
+    } else {
+        const uint32_t a = __builtin_amdgcn_alignbit(v[1], v[0], shift);
+        const uint32_t b = __builtin_amdgcn_alignbit(v[2], v[1], shift);
+        auto f = [](uint32_t h) { return F16 ? f16_bits_hw((uint16_t)h) : bf16_to_f32((uint16_t)h); };
+        return (f32x4){f(a & 0xffffu), f(a >> 16), f(b & 0xffffu), f(b >> 16)};
+    }
+}
+
+template <int MASK, bool F16>
+struct MaskAhead {
+    static constexpr int ES = MASK == 1 ? 4 : MASK == 3 ? 1 : 2;  // bytes of an element
+    static constexpr int W = MASK_W<MASK>;
+    typedef uint32_t quad __attribute__((ext_vector_type(W)));
+    MaskRow row;
+    __device__ __attribute__((always_inline)) inline MaskAhead(const MaskRef& m, int b, int h, int qi, int L, int S)
+        : row(m, ES, b, h, qi, L, S) {}
+    __device__ __attribute__((always_inline)) inline quad load(int key) const {
+        quad v{};
+#if __HIP_DEVICE_COMPILE__
+        const uint32_t o = row.off + (uint32_t)(key * ES);
+        if constexpr (W == 2) v = __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b64(row.r, o, 0, 0));
+        else if constexpr (W == 3) v = __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b96(row.r, o, 0, 0));
+        else v = __builtin_bit_cast(quad, __builtin_amdgcn_raw_buffer_load_b128(row.r, o, 0, 0));
+#else
+        (void)key;
+#endif
+        return v;
+    }
+    __device__ __attribute__((always_inline)) inline f32x4 values(quad v) const {
+        return mask_values<MASK, F16>(v, row.shift);
+    }
+};
+
+// Whether MaskAhead takes a mask of es-byte elements (aligned to es).
+inline bool mask_ahead(const MaskRef& m, int64_t L, int64_t S, int es) {
+    return m.sk == 1 && m.sl >= 0 && m.sl <= INT32_MAX && reinterpret_cast<uintptr_t>(m.p) % es == 0 &&
+           ((L - 1) * m.sl + S) * es <= INT32_MAX - 8;
+}
+
 // 16 bytes per lane from a raw buffer straight into LDS (buffer_load_dwordx4
 // ... lds): lane l's bytes land at lds_wave_base + 16*l, which must be
 // wave-uniform.

@@ -19,6 +19,7 @@ struct AnyArgs {
     float* part_o;     // BH * L * nsplit * D floats and
     float2* part_ml;   // BH * L * nsplit pairs
     int mk;            // mask kind: 0 none, 1 f32, 2 the input format, 3 bool
+    int mahead;        // its quads are loaded with their keys (mask_ahead)
     const void* mask;  // and its element strides over (B, Hq, L, S)
     int64_t msb, msh, msl, msk;
 };

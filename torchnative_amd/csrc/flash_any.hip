@@ -47,6 +47,15 @@ __device__ inline f32x4 any_mask_quad(int kind, const MaskRef& m, int64_t row, i
     return mask_quad<2, F16>(m, row, key, S);
 }
 
+// The same from a quad loaded ahead (MaskAhead), its format at run time.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <bool F16>
+__device__ inline f32x4 any_mask_values(int kind, u32x4 v, uint32_t shift) {
+    if (kind == 1) return mask_values<1, F16>(v, shift);
+    if (kind == 3) return mask_values<3, F16>(v, shift);
+    return mask_values<2, F16>(v, shift);
+}
+
 // f16: probabilities times 2^6 (at most 2^14 with the lazy rescale's slack),
 // so that they leave f16's normal range six powers of two later
 template <bool F16>
@@ -116,19 +125,53 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
         for (int i = 0; i < LPT; i++) rv.load16(voff[i], s + C::STAGE + (w * LPT + i) * 1024);
     };
 
+    // a stage's mask quads come with its K and V (four dwords whatever the
+    // format; past the plane they read as zeros)
+    const MaskRef mask{a.mask, a.msb, a.msh, a.msl, a.msk};
+    const int mes = a.mk == 1 ? 4 : a.mk == 3 ? 1 : 2;
+    [[maybe_unused]] const MaskRow mr(mask, mes, b, h, qi, a.L, a.S);
+    [[maybe_unused]] u32x4 mq[4] = {}, mcur[4];
+    auto mload = [&](int st) __attribute__((always_inline)) {
+#if __HIP_DEVICE_COMPILE__
+        if constexpr (MASKED) {
+            if (a.mahead) {
+#pragma unroll
+                for (int rq = 0; rq < 4; rq++)
+                    mq[rq] = __builtin_bit_cast(
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                   mr.r, mr.off + (uint32_t)((st * C::ROWS + kg * 32 + 8 * rq + 4 * hh) * mes), 0, 0));
+            }
+        }
+#endif
+    };
+
     f32x16 o[DT];
 #pragma unroll
     for (int i = 0; i < DT; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) o[i][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
-    if (st_lo < st_hi) issue(st_lo);
+    if (st_lo < st_hi) {
+        issue(st_lo);
+        mload(st_lo);
+    }
     for (int st = st_lo; st < st_hi; st++) {
         wait_vmcnt<0>();  // the only loads in flight are this stage's
+        if constexpr (MASKED) {
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                // the compiler's own wait falls here, where nothing is in flight
+                asm volatile("" : "+v"(mq[rq]));
+                mcur[rq] = mq[rq];
+            }
+        }
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (st + 1 < st_hi) issue(st + 1);  // into the stage read before the barrier
+        if (st + 1 < st_hi) {
+            issue(st + 1);  // into the stage read before the barrier
+            mload(st + 1);
+        }
         const int k0 = st * C::ROWS + kg * 32;
         if (k0 >= kend || (a.causal && qw0 + 31 < k0)) continue;
         const uint16_t* tK = reinterpret_cast<const uint16_t*>(ring + (st & 1) * 2 * C::STAGE);
@@ -150,8 +193,14 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
 #pragma unroll
         for (int r = 0; r < 16; r++) v[r] = acc[r] * a.sl2;
         if constexpr (MASKED) {
-            if (qi < a.L) {
-                const MaskRef mask{a.mask, a.msb, a.msh, a.msl, a.msk};
+            if (a.mahead) {
+#pragma unroll
+                for (int rq = 0; rq < 4; rq++) {
+                    const f32x4 mv = any_mask_values<F16>(a.mk, mcur[rq], mr.shift);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] + mv[e] * LOG2E;
+                }
+            } else if (qi < a.L) {
                 const int64_t mrow = (int64_t)b * mask.sb + (int64_t)h * mask.sh + (int64_t)qi * mask.sl;
 #pragma unroll
                 for (int rq = 0; rq < 4; rq++) {

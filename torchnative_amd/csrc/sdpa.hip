@@ -219,7 +219,7 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     const uint16_t* __restrict__ Qg, const uint16_t* __restrict__ Kg, const uint16_t* __restrict__ Vg, int Hq,
     int Hkv, int L, int S, float sl2, int causal, const FlashWork work, int nsplit, uint16_t* __restrict__ Og,
     float* __restrict__ lse, float* __restrict__ part_o, float2* __restrict__ part_ml, uint32_t* __restrict__ tickets,
-    const MaskRef mask) {
+    const MaskRef mask, int mahead) {
     constexpr int KG = FlashCfg<D>::KG;        // key groups
     constexpr int BKW = FlashCfg<D>::BKW;      // keys per wave tile
     constexpr int NH = BKW / 32;               // 32-key halves per wave tile
@@ -309,6 +309,24 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
         }
     };
 
+    // The mask quads of a stage are requested with its K and V. (Loaded where
+    // they are used, each wait for them also waited for the next stage's K and V,
+    // requested just before: 2 x 16 heads, 1000 keys, D 128, f16, took 46 us with a
+    // key mask and 56 with a full one, against 35.5 without; now 39 and 41. 1001 keys,
+    // whose rows lie at any alignment, bf16: 109 with a full mask, now 34.)
+    using MA = MaskAhead<MASK == 0 ? 3 : MASK, F16>;
+    [[maybe_unused]] const MA ma(mask, b, h, qi, L, S);
+    [[maybe_unused]] typename MA::quad mq[2][4 * NH];
+    auto mload = [&](auto sc, int st) __attribute__((always_inline)) {
+        if constexpr (MASK != 0) {
+            if (mahead) {
+#pragma unroll
+                for (int rq = 0; rq < 4 * NH; rq++)
+                    mq[decltype(sc)::value][rq] = ma.load(k_lo + st * ROWS + kg * BKW + 8 * rq + 4 * hh);
+            }
+        }
+    };
+
     f32x16 o[D / 32];
 #pragma unroll
     for (int i = 0; i < D / 32; i++)
@@ -319,6 +337,7 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     issue(I0{}, 0);  // nst >= 1: every item has at least one key
+    mload(I0{}, 0);
 
     // ring stage sc holds stage st: wait for it, open the other stage (read in
     // the previous step) to the next stage's loads, compute this wave's tile
@@ -330,7 +349,10 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (st + 1 < nst) issue(std::integral_constant<int, 1 - decltype(sc)::value>{}, st + 1);
+        if (st + 1 < nst) {
+            issue(std::integral_constant<int, 1 - decltype(sc)::value>{}, st + 1);
+            mload(std::integral_constant<int, 1 - decltype(sc)::value>{}, st + 1);
+        }
 
         const int k0 = k_lo + st * ROWS + kg * BKW;
         // past the item's keys, or every query of the wave precedes the tile
@@ -380,7 +402,14 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
             if constexpr (MASK != 0) {
                 // scores to log2 units with the mask added: raw*scale*log2e + mask*log2e;
                 // from here on the scale is 1
-                if (qi < L) {
+                if (mahead) {
+#pragma unroll
+                    for (int rq = 0; rq < 4; rq++) {
+                        const f32x4 mv = ma.values(mq[decltype(sc)::value][4 * s2 + rq]);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] * sl2 + mv[e] * LOG2E;
+                    }
+                } else if (qi < L) {
                     const int64_t mrow = (int64_t)b * mask.sb + (int64_t)h * mask.sh + (int64_t)qi * mask.sl;
 #pragma unroll
                     for (int rq = 0; rq < 4; rq++) {
@@ -701,7 +730,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                                               float sl2, int causal, const SkGeo geo,
                                               float* __restrict__ Og, float* __restrict__ lse,
                                               float* __restrict__ part_o, float2* __restrict__ part_ml,
-                                              uint32_t* __restrict__ tickets, const MaskRef mask) {
+                                              uint32_t* __restrict__ tickets, const MaskRef mask, int mahead) {
     constexpr int BQ = PF_BQ;
     constexpr int RS = D + 4;
     constexpr int CH = (BK * D / 4) / PF_THREADS;  // float4 chunks of K (and of V) per thread
@@ -750,6 +779,10 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                 for (int i = 0; i < 4; i++) o[e][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
             float m = -INFINITY, l = 0.0f;
 
+            using MA = MaskAhead<MASK == 0 ? 3 : MASK, false>;
+            [[maybe_unused]] const MA ma(mask, b, h, qi, L, S);
+            [[maybe_unused]] typename MA::quad mq[BK / 16];
+
             float4 kr[CH], vr[CH];
             auto gload = [&](int k0) {
         #pragma unroll
@@ -785,6 +818,13 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
             for (int t = t_begin; t < t_end; t++) {
                 const int buf = (t - t_begin) & 1;
                 const int k0 = t * BK;
+                // before the next tile's K and V: waiting for it leaves those in flight
+                if constexpr (MASK != 0) {
+                    if (mahead) {
+        #pragma unroll
+                        for (int kt = 0; kt < BK / 16; kt++) mq[kt] = ma.load(k0 + 16 * kt + 4 * g);
+                    }
+                }
                 if (t + 1 < t_end) gload(k0 + BK);
 
                 f32x4 s[BK / 16];
@@ -810,7 +850,14 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                 }
                 if constexpr (MASK != 0) {
                     // scores to log2 units with the mask added; from here on the scale is 1
-                    if (qi < L) {
+                    if (mahead) {
+        #pragma unroll
+                        for (int kt = 0; kt < BK / 16; kt++) {
+                            const f32x4 mv = ma.values(mq[kt]);
+        #pragma unroll
+                            for (int r = 0; r < 4; r++) s[kt][r] = s[kt][r] * sl2 + mv[r] * LOG2E;
+                        }
+                    } else if (qi < L) {
                         const int64_t mrow = (int64_t)b * mask.sb + (int64_t)h * mask.sh + (int64_t)qi * mask.sl;
         #pragma unroll
                         for (int kt = 0; kt < BK / 16; kt++) {
@@ -2352,6 +2399,7 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
     hipStream_t st = (hipStream_t)stream;
     const int c = is_causal ? 1 : 0;
     const int64_t rows = B * Hq * L;
+    const int mahead = mk && mask_ahead(mref, L, S, mk == 1 ? 4 : mk == 3 ? 1 : 2);
     // the MFMA kernels take the row maximum of the unscaled scores (right for
     // scale >= 0) and exist for head dims 64 and 128; anything else runs on
     // the plain kernel
@@ -2373,6 +2421,7 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
             a.causal = c;
             a.nsplit = 1;
             a.mk = mk;
+            a.mahead = mahead;
             a.mask = attn_mask;
             a.msb = mref.sb, a.msh = mref.sh, a.msl = mref.sl, a.msk = mref.sk;
             if (flash_any_takes(a)) {
@@ -2465,7 +2514,7 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
 #define TN_FLASH(DD, MK, H)                                                                                      \
     hipLaunchKernelGGL((k_flash16<DD, MK, H>), dim3((unsigned)nitems), dim3(128 * FlashCfg<DD>::KG), 0, st, qq, kk, \
                        vv, (int)Hq, (int)Hkv, (int)L, (int)S, sl2, c, work, nsplit, oo, lse, part_o, part_ml, tick,   \
-                       mref)
+                       mref, mahead)
 #define TN_FLASH_MK(DD, H)              \
     do {                                \
         if (mk == 0) TN_FLASH(DD, 0, H); \
@@ -2521,10 +2570,18 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
         auto kk = static_cast<const float*>(k);
         auto vv = static_cast<const float*>(v);
         auto oo = static_cast<float*>(out);
+        // Aligned mask quads are as fast loaded where they are used (8 heads, 700
+        // keys, D 64, us: 26.7, 27.3 ahead); others take four loads an element
+        // there (701 keys: 30.2, 27.4 ahead).
+        const int me = mk == 1 ? 4 : 1;
+        const bool quads = mref.sk == 1 && S % 4 == 0 && mref.sl % 4 == 0 && mref.sh % 4 == 0 && mref.sb % 4 == 0 &&
+                           reinterpret_cast<uintptr_t>(attn_mask) % (4 * me) == 0;
+        const int ahead = mahead && !quads;
         // an f32 query takes an f32 mask (mk 1) or a bool one (mk 3)
 #define TN_FA(DD, BKK, MK)                                                                                       \
     hipLaunchKernelGGL((k_fa_f32<DD, BKK, MK>), dim3((unsigned)geo.G), dim3(PF_THREADS), 0, st, qq, kk, vv,      \
-                       (int)Hq, (int)Hkv, (int)L, (int)S, sl2, c, geo, oo, lse, part_o, part_ml, tick, mref)
+                       (int)Hq, (int)Hkv, (int)L, (int)S, sl2, c, geo, oo, lse, part_o, part_ml, tick, mref,   \
+                       ahead)
         if (D == 64) {
             if (mk == 1) TN_FA(64, 64, 1);
             else if (mk == 3) TN_FA(64, 64, 3);
