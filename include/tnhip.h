@@ -257,10 +257,11 @@ tn_status tn_dense_linear(void* stream, const float* x, int64_t m, int64_t k, co
  * f32, aten.rs:10196-10213); a bf16 or f16 run narrows the probabilities to
  * its dtype between the two products, as upstream's blocked kernel does
  * (flash.rs:503-516), and the output RNE.
- * Head dims 64 and 128 with scale >= 0 run on MFMA kernels; so do 16-bit
- * inputs at any other multiple of 8 up to 256, or with a negative scale (the
- * probabilities as a sum of two 16-bit parts there). What is left, and rows
- * that are not 16-byte aligned, runs on a plain f32 kernel (f32
+ * Head dims 64 and 128 with scale > 0 run on MFMA kernels; so do 16-bit inputs
+ * at any other multiple of 8 up to 256, or with another scale (the
+ * probabilities as a sum of two 16-bit parts there), and f32 ones at any
+ * multiple of 4 (unless a capture could not grow the stream's buffers). What is
+ * left, and rows that are not 16-byte aligned, runs on a plain f32 kernel (f32
  * probabilities); a head dim past 256 is refused by name. */
 tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, const void* v,
                       int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t S, int64_t D,
@@ -280,9 +281,10 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
  *   max_len: host upper bound of lens (sizes the split-KV grid);
  *   lse nullable f32 [B, Hq].
  * Head dims 64 and 128: split-KV with a combine pass, the partials in the
- * library workspace; so do 16-bit caches at any other multiple of 8 up to 256
- * (unsplit where a capture could not grow the workspace); otherwise a head dim
- * up to 256 runs on the plain kernel (one workgroup per (sequence, head)). A sequence of length 0 gives NaN out
+ * library workspace; so do 16-bit caches at any other multiple of 8 and f32
+ * ones at any other multiple of 4 up to 256 (unsplit where a capture could not
+ * grow the workspace); otherwise a head dim up to 256 runs on the plain kernel
+ * (one workgroup per (sequence, head)). A sequence of length 0 gives NaN out
  * and -inf lse. */
 tn_status tn_sdpa_decode(void* stream, int dtype, const void* q, const void* k_cache,
                          const void* v_cache, int64_t B, int64_t Hq, int64_t Hkv, int64_t cap,

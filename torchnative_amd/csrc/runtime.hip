@@ -148,6 +148,22 @@ tn_status tickets(hipStream_t stream, size_t n, uint32_t** out) {
     return TN_OK;
 }
 
+tn_status tickets_or_none(hipStream_t stream, size_t n, uint32_t** out) {
+    *out = nullptr;
+    int dev = 0;
+    TN_HIP(hipGetDevice(&dev));
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mu);
+        const Workspace& w = g_ws[{dev, stream}];
+        if (w.ntickets < n) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            TN_HIP(hipStreamIsCapturing(stream, &cs));
+            if (cs != hipStreamCaptureStatusNone) return TN_OK;
+        }
+    }
+    return tickets(stream, n, out);
+}
+
 namespace {
 struct OccKey {
     int dev;

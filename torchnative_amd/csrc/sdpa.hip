@@ -32,6 +32,7 @@
 
 #include "tn_common.h"
 #include "attn_common.h"
+#include "decode_any.h"
 #include "flash_any.h"
 #include "skgeo.h"
 
@@ -723,15 +724,21 @@ constexpr int PF_BQ = 16 * PF_WAVES, PF_BK = 64;
 // ---------------------------------------------------------------------------
 
 // MASK: 1 adds an f32 mask, 3 a bool one (MaskRef), to the scaled scores
-// (aten.rs:10383-10389)
-template <int D, int BK, int MASK = 0>
+// (aten.rs:10383-10389). ANY: a head dim Dr below the padded D (a multiple of
+// four; the columns past it are zeros in registers and LDS and are not stored),
+// and q times qsign, the sign of the scale, so that the maximum is that of
+// products times |scale|. us on the plain kernel -> here: 4 heads, 1024 causal keys, head
+// dim 96: 518 -> 57.5; 2 x 8 heads, 200 queries, 1000 keys, head dim 72: 667 -> 38;
+// 2 x 8 heads, 300 causal keys, head dim 256: 481 -> 45.
+template <int D, int BK, int MASK = 0, bool ANY = false>
 __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__ Qg, const float* __restrict__ Kg,
                                               const float* __restrict__ Vg, int Hq, int Hkv, int L, int S,
                                               float sl2, int causal, const SkGeo geo,
                                               float* __restrict__ Og, float* __restrict__ lse,
                                               float* __restrict__ part_o, float2* __restrict__ part_ml,
-                                              uint32_t* __restrict__ tickets, const MaskRef mask, int mahead) {
+                                              uint32_t* __restrict__ tickets, const MaskRef mask, int mahead, int Dr, float qsign) {
     constexpr int BQ = PF_BQ;
+    const int DM = ANY ? Dr : D;  // the head dim in memory
     constexpr int RS = D + 4;
     constexpr int CH = (BK * D / 4) / PF_THREADS;  // float4 chunks of K (and of V) per thread
     static_assert(CH * PF_THREADS == BK * D / 4, "tile staging");
@@ -752,9 +759,9 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
         const int kvh = h / (Hq / Hkv);
         const int q0 = qt * BQ;
         const int qi = q0 + w * 16 + lq;
-        const float* qp = Qg + ((int64_t)b * Hq + h) * L * D;
-        const float* kp = Kg + ((int64_t)b * Hkv + kvh) * S * D;
-        const float* vp = Vg + ((int64_t)b * Hkv + kvh) * S * D;
+        const float* qp = Qg + ((int64_t)b * Hq + h) * L * DM;
+        const float* kp = Kg + ((int64_t)b * Hkv + kvh) * S * DM;
+        const float* vp = Vg + ((int64_t)b * Hkv + kvh) * S * DM;
 
             // q[16g + c] for the D/16 row slices of 16: slice e holds d = 64e + 16g + c
             constexpr int DS = D / 64;  // 64-wide slices of the head dim
@@ -765,7 +772,11 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
         #pragma unroll
                 for (int c4 = 0; c4 < 4; c4++) {
                     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (qi < L) v = *reinterpret_cast<const float4*>(qp + (int64_t)qi * D + 64 * e + 16 * g + 4 * c4);
+                    const int d = 64 * e + 16 * g + 4 * c4;
+                    if (qi < L && (!ANY || d < DM)) {
+                        v = *reinterpret_cast<const float4*>(qp + (int64_t)qi * DM + d);
+                        if constexpr (ANY) v = make_float4(v.x * qsign, v.y * qsign, v.z * qsign, v.w * qsign);
+                    }
                     qf[e][4 * c4] = v.x;
                     qf[e][4 * c4 + 1] = v.y;
                     qf[e][4 * c4 + 2] = v.z;
@@ -790,9 +801,9 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                     const int c = tid + it * PF_THREADS;
                     const int r = c / (D / 4), part = c % (D / 4);
                     kr[it] = vr[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (k0 + r < S) {
-                        kr[it] = *reinterpret_cast<const float4*>(kp + (int64_t)(k0 + r) * D + part * 4);
-                        vr[it] = *reinterpret_cast<const float4*>(vp + (int64_t)(k0 + r) * D + part * 4);
+                    if (k0 + r < S && (!ANY || part * 4 < DM)) {
+                        kr[it] = *reinterpret_cast<const float4*>(kp + (int64_t)(k0 + r) * DM + part * 4);
+                        vr[it] = *reinterpret_cast<const float4*>(vp + (int64_t)(k0 + r) * DM + part * 4);
                     }
                 }
             };
@@ -933,13 +944,14 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
             if (qi >= L) return;
             const int64_t row = bh * L + qi;
             const float inv = 1.0f / l;
-            float* op = Og + row * D;
+            float* op = Og + row * DM;
 #pragma unroll
             for (int e = 0; e < DS; e++)
 #pragma unroll
                 for (int r = 0; r < 4; r++)
-                    *reinterpret_cast<float4*>(op + 64 * e + 16 * g + 4 * r) =
-                        make_float4(o[e][0][r] * inv, o[e][1][r] * inv, o[e][2][r] * inv, o[e][3][r] * inv);
+                    if (!ANY || 64 * e + 16 * g + 4 * r < DM)
+                        *reinterpret_cast<float4*>(op + 64 * e + 16 * g + 4 * r) =
+                            make_float4(o[e][0][r] * inv, o[e][1][r] * inv, o[e][2][r] * inv, o[e][3][r] * inv);
             if (lse && g == 0) lse[row] = m == -INFINITY ? NAN : m * LN2 + logf(l);
             return;
         }
@@ -1000,7 +1012,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
             const int rr = 16 * wv + (ln & 15);
             const int c4 = 64 * (k >> 2) + 16 * (ln >> 4) + 4 * (k & 3);
             const int qrow = qt * BQ + rr;
-            if (qrow >= L) continue;
+            if (qrow >= L || (ANY && c4 >= DM)) continue;
             auto prow_of = [&](int i) { return (uint32_t)((i == 0 ? s_lo : 2 * (g_lo + i)) * BQ + rr); };
             auto slot_of = [&](int i) { return (uint32_t)(i == 0 ? s_lo : 2 * (g_lo + i)); };
             typedef float f32x2_t __attribute__((ext_vector_type(2)));
@@ -1039,7 +1051,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
             for (int i = CMAX; i < np; i++) add(ld_ml(i), ld_o(i));
             const float inv = 1.0f / tl;
             const int64_t row = bh * L + qrow;
-            *reinterpret_cast<float4*>(Og + row * D + c4) = make_float4(a0 * inv, a1 * inv, a2 * inv, a3 * inv);
+            *reinterpret_cast<float4*>(Og + row * DM + c4) = make_float4(a0 * inv, a1 * inv, a2 * inv, a3 * inv);
             if (lse && c4 == 0) lse[row] = mm == -INFINITY ? NAN : mu * LN2 + logf(tl);
         }
 #endif
@@ -2023,10 +2035,10 @@ tn_status decode_check(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t ca
     return TN_OK;
 }
 
-// Decode attention at the head dims other than 64 and 128: flash_any for
-// 16-bit caches (the partials, if given, hold max_split splits of B * Hq
-// rows), otherwise the plain kernel, one query row per (sequence, head) over
-// the cache's cap rows.
+// Decode attention at the head dims other than 64 and 128: flash_any for 16-bit
+// caches and decode_any_f32 for f32 ones (the partials, if given, hold max_split
+// splits of B * Hq rows), otherwise the plain kernel, one query row per
+// (sequence, head) over the cache's cap rows.
 static tn_status decode_any(hipStream_t st, int dtype, const void* q, const void* k_cache, const void* v_cache, int64_t B,
                             int64_t Hq, int64_t Hkv, int64_t cap, int64_t D, const int32_t* lens, int64_t max_len,
                             double sc, void* out, float* lse, float* part_o, float2* part_ml, int max_split) {
@@ -2038,6 +2050,12 @@ static tn_status decode_any(hipStream_t st, int dtype, const void* q, const void
             a.part_ml = part_ml;
             return flash_any_launch(st, dtype == TN_F16, a);
         }
+    }
+    if (dtype == TN_F32 && decode_any_f32_takes(Hq, D)) {
+        const int ns = part_o ? std::min(max_split, decode_any_f32_splits(B, Hq, Hkv, D, max_len)) : 1;
+        return decode_any_f32(st, static_cast<const float*>(q), static_cast<const float*>(k_cache),
+                              static_cast<const float*>(v_cache), B, Hq, Hkv, cap, D, lens, max_len, sc,
+                              static_cast<float*>(out), lse, part_o, part_ml, ns);
     }
     const dim3 grid(1u, (unsigned)Hq, (unsigned)B);
     if (dtype == TN_F32)
@@ -2340,6 +2358,90 @@ tn_status flash_plan(hipStream_t st, int64_t B, int64_t Hq, int64_t L, int64_t S
 
 using namespace tn;
 
+// The f32 flash kernel. any: head dims other than 64 and 128 and scales of at
+// most zero, on the padded variants; there *taken is false, and nothing was launched, where
+// a capture could not grow the stream's buffers.
+static tn_status flash_f32(hipStream_t st, bool any, const void* q, const void* k, const void* v, int64_t B, int64_t Hq,
+                           int64_t Hkv, int64_t L, int64_t S, int64_t D, float sl2, int c, int mk, const MaskRef& mref,
+                           bool mahead, void* out, float* lse, bool* taken) {
+    if (taken) *taken = true;
+    const int DP = D <= 64 ? 64 : D <= 128 ? 128 : 256;  // the kernel's head dim
+    const int bk = DP == 256 ? 16 : DP == 128 ? 32 : PF_BK;
+    // the stream-K grid: one workgroup per resident slot, at most one per unit
+    int slots = 0;
+    {
+        const void* kern = DP == 256 ? reinterpret_cast<const void*>(&k_fa_f32<256, 16, 0, true>)
+                           : any ? (DP == 64 ? reinterpret_cast<const void*>(&k_fa_f32<64, 64, 0, true>)
+                                             : reinterpret_cast<const void*>(&k_fa_f32<128, 32, 0, true>))
+                                 : (DP == 64 ? reinterpret_cast<const void*>(&k_fa_f32<64, 64, 0>)
+                                             : reinterpret_cast<const void*>(&k_fa_f32<128, 32, 0>));
+        tn_status sp = resident_workgroups(kern, PF_THREADS, 0, &slots);
+        if (sp != TN_OK) return sp;
+    }
+    SkGeo geo;
+    geo.nqb = (int)cdiv(L, PF_BQ);
+    geo.NS = (int)cdiv(S, bk);
+    geo.c = PF_BQ / bk;
+    geo.causal = c;
+    geo.Tbh = geo.P(geo.nqb);
+    geo.T = B * Hq * geo.Tbh;
+    geo.G = std::min<int64_t>(std::max(slots, 1), geo.T);
+    float* part_o = nullptr;
+    float2* part_ml = nullptr;
+    uint32_t* tick = nullptr;
+    if (geo.G > 1) {
+        const size_t po = (size_t)(2 * geo.G) * PF_BQ * DP * sizeof(float);
+        const size_t pm = (size_t)(2 * geo.G) * PF_BQ * sizeof(float2);
+        void* ws = nullptr;
+        TN_TRY((any ? workspace_or_none : workspace)(st, po + pm, &ws));
+        part_o = static_cast<float*>(ws);
+        part_ml = reinterpret_cast<float2*>(static_cast<char*>(ws) + po);
+        // one counter per (batch, head, query block); only cut blocks take tickets
+        if (ws) TN_TRY((any ? tickets_or_none : tickets)(st, (size_t)(B * Hq) * (size_t)geo.nqb, &tick));
+        if (!tick) {
+            *taken = false;
+            return TN_OK;
+        }
+    }
+    {
+        auto qq = static_cast<const float*>(q);
+        auto kk = static_cast<const float*>(k);
+        auto vv = static_cast<const float*>(v);
+        auto oo = static_cast<float*>(out);
+        // Aligned mask quads are as fast loaded where they are used (8 heads, 700
+        // keys, D 64, us: 26.7, 27.3 ahead); others take four loads an element
+        // there (701 keys: 30.2, 27.4 ahead).
+        const int me = mk == 1 ? 4 : 1;
+        const bool quads = mref.sk == 1 && S % 4 == 0 && mref.sl % 4 == 0 && mref.sh % 4 == 0 && mref.sb % 4 == 0 &&
+                           reinterpret_cast<uintptr_t>(mref.p) % (4 * me) == 0;
+        const int ahead = mahead && !quads;
+        // an f32 query takes an f32 mask (mk 1) or a bool one (mk 3)
+#define TN_FA(DD, BKK, MK, ANY)                                                                                  \
+    hipLaunchKernelGGL((k_fa_f32<DD, BKK, MK, ANY>), dim3((unsigned)geo.G), dim3(PF_THREADS), 0, st, qq, kk, vv,      \
+                       (int)Hq, (int)Hkv, (int)L, (int)S, asl2, c, geo, oo, lse, part_o, part_ml, tick, mref,   \
+                       ahead, (int)D, qsign)
+#define TN_FA_MK(DD, BKK, ANY)                \
+    do {                                      \
+        if (mk == 1) TN_FA(DD, BKK, 1, ANY);  \
+        else if (mk == 3) TN_FA(DD, BKK, 3, ANY); \
+        else TN_FA(DD, BKK, 0, ANY);          \
+    } while (0)
+        // at most zero only if any; a zero scale makes q zeros, as hidden keys'
+        // -inf is not to be multiplied by it
+        const float qsign = sl2 > 0.0f ? 1.0f : sl2 < 0.0f ? -1.0f : 0.0f;
+        const float asl2 = sl2 == 0.0f ? 1.0f : std::fabs(sl2);
+        if (DP == 256) TN_FA_MK(256, 16, true);
+        else if (any && DP == 64) TN_FA_MK(64, 64, true);
+        else if (any) TN_FA_MK(128, 32, true);
+        else if (DP == 64) TN_FA_MK(64, 64, false);
+        else TN_FA_MK(128, 32, false);
+#undef TN_FA_MK
+#undef TN_FA
+        TN_LAUNCHED();
+    }
+    return TN_OK;
+}
+
 extern "C" {
 
 tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, const void* v, int64_t B, int64_t Hq,
@@ -2400,10 +2502,11 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
     const int c = is_causal ? 1 : 0;
     const int64_t rows = B * Hq * L;
     const int mahead = mk && mask_ahead(mref, L, S, mk == 1 ? 4 : mk == 3 ? 1 : 2);
-    // the MFMA kernels take the row maximum of the unscaled scores (right for
-    // scale >= 0) and exist for head dims 64 and 128; anything else runs on
-    // the plain kernel
-    if ((D != 64 && D != 128) || sc < 0.0 || dtype == TN_F64) {
+    // the kernels for head dims 64 and 128 take the row maximum of the unscaled
+    // scores, hidden ones -inf (right for scale > 0); anything else runs on flash_any (16-bit) or
+    // the padded f32 kernel, and what those do not take (f64, head dims that are
+    // no multiple of 8 or 4, unaligned pointers) on the plain kernel
+    if ((D != 64 && D != 128) || sl2 <= 0.0f || dtype == TN_F64) {
         if (dtype == TN_BF16 || dtype == TN_F16) {
             AnyArgs a{};
             a.q = static_cast<const uint16_t*>(q);
@@ -2440,6 +2543,12 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
                 }
                 return flash_any_launch(st, dtype == TN_F16, a);
             }
+        }
+        if (dtype == TN_F32 && D % 4 == 0 &&
+            ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0) {
+            bool taken = false;
+            TN_TRY(flash_f32(st, true, q, k, v, B, Hq, Hkv, L, S, D, sl2, c, mk, mref, mahead, out, lse, &taken));
+            if (taken) return TN_OK;
         }
         const dim3 grid((unsigned)cdiv(L, ANY_BQ), (unsigned)Hq, (unsigned)B);
         const int et = dtype == TN_F32 ? 0 : dtype == TN_BF16 ? 1 : dtype == TN_F16 ? 2 : 3;
@@ -2533,68 +2642,7 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
         TN_LAUNCHED();
         return TN_OK;
     }
-    const int bk = (D == 128) ? 32 : PF_BK;
-    // the stream-K grid: one workgroup per resident slot, at most one per unit
-    int slots = 0;
-    {
-        tn_status sp = resident_workgroups(D == 64 ? reinterpret_cast<const void*>(&k_fa_f32<64, 64, 0>)
-                                                    : reinterpret_cast<const void*>(&k_fa_f32<128, 32, 0>),
-                                           PF_THREADS, 0, &slots);
-        if (sp != TN_OK) return sp;
-    }
-    SkGeo geo;
-    geo.nqb = (int)cdiv(L, PF_BQ);
-    geo.NS = (int)cdiv(S, bk);
-    geo.c = PF_BQ / bk;
-    geo.causal = c;
-    geo.Tbh = geo.P(geo.nqb);
-    geo.T = B * Hq * geo.Tbh;
-    geo.G = std::min<int64_t>(std::max(slots, 1), geo.T);
-    float* part_o = nullptr;
-    float2* part_ml = nullptr;
-    uint32_t* tick = nullptr;
-    if (geo.G > 1) {
-        const size_t po = (size_t)(2 * geo.G) * PF_BQ * D * sizeof(float);
-        const size_t pm = (size_t)(2 * geo.G) * PF_BQ * sizeof(float2);
-        void* ws = nullptr;
-        tn_status s = workspace(st, po + pm, &ws);
-        if (s != TN_OK) return s;
-        part_o = static_cast<float*>(ws);
-        part_ml = reinterpret_cast<float2*>(static_cast<char*>(ws) + po);
-        // one counter per (batch, head, query block); only cut blocks take tickets
-        s = tickets(st, (size_t)(B * Hq) * (size_t)geo.nqb, &tick);
-        if (s != TN_OK) return s;
-    }
-    {
-        auto qq = static_cast<const float*>(q);
-        auto kk = static_cast<const float*>(k);
-        auto vv = static_cast<const float*>(v);
-        auto oo = static_cast<float*>(out);
-        // Aligned mask quads are as fast loaded where they are used (8 heads, 700
-        // keys, D 64, us: 26.7, 27.3 ahead); others take four loads an element
-        // there (701 keys: 30.2, 27.4 ahead).
-        const int me = mk == 1 ? 4 : 1;
-        const bool quads = mref.sk == 1 && S % 4 == 0 && mref.sl % 4 == 0 && mref.sh % 4 == 0 && mref.sb % 4 == 0 &&
-                           reinterpret_cast<uintptr_t>(attn_mask) % (4 * me) == 0;
-        const int ahead = mahead && !quads;
-        // an f32 query takes an f32 mask (mk 1) or a bool one (mk 3)
-#define TN_FA(DD, BKK, MK)                                                                                       \
-    hipLaunchKernelGGL((k_fa_f32<DD, BKK, MK>), dim3((unsigned)geo.G), dim3(PF_THREADS), 0, st, qq, kk, vv,      \
-                       (int)Hq, (int)Hkv, (int)L, (int)S, sl2, c, geo, oo, lse, part_o, part_ml, tick, mref,   \
-                       ahead)
-        if (D == 64) {
-            if (mk == 1) TN_FA(64, 64, 1);
-            else if (mk == 3) TN_FA(64, 64, 3);
-            else TN_FA(64, 64, 0);
-        } else {
-            if (mk == 1) TN_FA(128, 32, 1);
-            else if (mk == 3) TN_FA(128, 32, 3);
-            else TN_FA(128, 32, 0);
-        }
-#undef TN_FA
-        TN_LAUNCHED();
-    }
-    return TN_OK;
+    return flash_f32(st, false, q, k, v, B, Hq, Hkv, L, S, D, sl2, c, mk, mref, mahead, out, lse, nullptr);
 }
 
 }  // extern "C"
@@ -2620,15 +2668,17 @@ tn_status decode_entry(void* stream, int dtype, const void* q, const void* k_cac
         if (dtype != TN_F32) {
             const AnyArgs a = decode_any_args(q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse);
             if (flash_any_takes(a)) ns = flash_any_splits(a);
-            if (ns > 1) {
-                // as many splits as the no-alloc entry's array holds, in either
-                // entry (they give the same bits); none where a capture could not
-                // grow the stream's workspace
-                const size_t one = (size_t)B * Hq * (D * sizeof(float) + sizeof(float2));
-                ns = (int)std::min<size_t>(ns, DECODE_SCRATCH_BYTES / one);
-                po = (size_t)B * Hq * ns * D * sizeof(float);
-                if (ns > 1) TN_TRY((get == workspace ? workspace_or_none : get)(st, one * ns, &ws));
-            }
+        } else if (decode_any_f32_takes(Hq, D)) {
+            ns = decode_any_f32_splits(B, Hq, Hkv, D, max_len);
+        }
+        if (ns > 1) {
+            // as many splits as the no-alloc entry's array holds, in either
+            // entry (they give the same bits); none where a capture could not
+            // grow the stream's workspace
+            const size_t one = (size_t)B * Hq * (D * sizeof(float) + sizeof(float2));
+            ns = (int)std::min<size_t>(ns, DECODE_SCRATCH_BYTES / one);
+            po = (size_t)B * Hq * ns * D * sizeof(float);
+            if (ns > 1) TN_TRY((get == workspace ? workspace_or_none : get)(st, one * ns, &ws));
         }
         return decode_any(st, dtype, q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse,
                           static_cast<float*>(ws), ws ? reinterpret_cast<float2*>(static_cast<char*>(ws) + po) : nullptr,

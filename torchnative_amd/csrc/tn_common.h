@@ -40,6 +40,8 @@ tn_status workspace_or_none(hipStream_t stream, size_t bytes, void** out);
 // (cleared on the stream at allocation). A kernel that takes tickets from it
 // must leave every counter at zero again when it ends.
 tn_status tickets(hipStream_t stream, size_t n, uint32_t** out);
+// As workspace_or_none.
+tn_status tickets_or_none(hipStream_t stream, size_t n, uint32_t** out);
 // Workgroups of `kernel` (block threads, lds dynamic bytes) that the current
 // device holds at once: the size of a persistent grid, all of whose
 // workgroups must be resident from the start. Cached per (device, kernel,
