@@ -27,11 +27,6 @@ __device__ inline uint32_t pack2_bf16_hw(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
 }
 
-// the same narrowing spelled out (reduced.rs:161-218: RNE, NaN quieted), for outputs
-__device__ inline uint32_t pack2_bf16(float a, float b) {
-    return (uint32_t)bf16_from_f32(a) | ((uint32_t)bf16_from_f32(b) << 16);
-}
-
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // The 16-bit storage formats of the prefill kernel: bf16 or f16 inputs, the
@@ -47,15 +42,11 @@ struct El<false> {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
     static __device__ inline uint32_t pack_p(float a, float b) { return pack2_bf16_hw(a, b); }
-    static __device__ inline uint32_t pack_out(float a, float b) { return pack2_bf16(a, b); }
-    // pack_out's bits through v_cvt_pk_bf16_f32 (round to nearest even, as
-    // bf16_from_f32 for every number), with a NaN given bf16_from_f32's
-    // quieted payload
-    static __device__ inline uint32_t pack_out_hw(float a, float b) {
-        uint32_t r = pack2_bf16_hw(a, b);
-        if (a != a) r = (r & 0xffff0000u) | ((__float_as_uint(a) >> 16) | 0x40u);
-        if (b != b) r = (r & 0xffffu) | (((__float_as_uint(b) >> 16) | 0x40u) << 16);
-        return r;
+    // outputs, any float (bf16_from_f32's bits)
+    static __device__ inline uint32_t pack_out(float a, float b) {
+        const uint32_t r = pack2_bf16_hw(a, b);
+        const uint32_t lo = a != a ? bf16_nan_bits(a) : r, hi = b != b ? bf16_nan_bits(b) : r >> 16;
+        return (lo & 0xffffu) | (hi << 16);
     }
     static __device__ inline float widen(uint16_t h) { return bf16_to_f32(h); }
     static __device__ inline f32x4 mfma16(v8 a, v8 b, f32x4 c) {
@@ -76,17 +67,11 @@ struct El<true> {
     static __device__ inline uint32_t pack_p(float a, float b) {
         return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, v2));
     }
+    // outputs, any float (f16_from_f32's bits)
     static __device__ inline uint32_t pack_out(float a, float b) {
-        return (uint32_t)f16_from_f32(a) | ((uint32_t)f16_from_f32(b) << 16);
-    }
-    // pack_out's bits through v_cvt_f16_f32 (equal to f16_from_f32 for every
-    // number, subnormals and overflow included), with a NaN given
-    // f16_from_f32's quieted payload
-    static __device__ inline uint32_t pack_out_hw(float a, float b) {
-        uint32_t r = pack_p(a, b);
-        if (a != a) r = (r & 0xffff0000u) | f16_from_f32(a);
-        if (b != b) r = (r & 0xffffu) | ((uint32_t)f16_from_f32(b) << 16);
-        return r;
+        const uint32_t r = pack_p(a, b);
+        const uint32_t lo = a != a ? f16_nan_bits(a) : r, hi = b != b ? f16_nan_bits(b) : r >> 16;
+        return (lo & 0xffffu) | (hi << 16);
     }
     static __device__ inline float widen(uint16_t h) { return f16_to_f32(h); }
     static __device__ inline f32x4 mfma16(v8 a, v8 b, f32x4 c) {

@@ -406,8 +406,8 @@ template <int WT>
 __global__ void k_dense_store(const float* __restrict__ x, int64_t count, void* __restrict__ out) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
         if constexpr (WT == TN_F32) reinterpret_cast<float*>(out)[i] = x[i];
-        else if constexpr (WT == TN_F16) reinterpret_cast<uint16_t*>(out)[i] = f16_from_f32(x[i]);
-        else reinterpret_cast<uint16_t*>(out)[i] = bf16_from_f32(x[i]);
+        else if constexpr (WT == TN_F16) reinterpret_cast<uint16_t*>(out)[i] = f16_out(x[i]);
+        else reinterpret_cast<uint16_t*>(out)[i] = bf16_out(x[i]);
     }
 }
 

@@ -382,7 +382,7 @@ __global__ __launch_bounds__(FA_NT) void k_fa64(const uint16_t* __restrict__ Qg,
             const float inv = __builtin_amdgcn_rcpf(tl);
             const int64_t row = (int64_t)bh * L + qrow;
             *reinterpret_cast<uint2*>(Og + row * D + 4 * c4) =
-                make_uint2(E::pack_out_hw(a0 * inv, a1 * inv), E::pack_out_hw(a2 * inv, a3 * inv));
+                make_uint2(E::pack_out(a0 * inv, a1 * inv), E::pack_out(a2 * inv, a3 * inv));
             if (lse && c4 == 0) lse[row] = mm == -INFINITY ? NAN : mm * LN2 + logf(tl);
         }
     }

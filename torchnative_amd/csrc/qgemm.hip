@@ -307,7 +307,7 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
                 if (bias) v = v + bv;
                 if (resid) v = resid[(int64_t)m * N + n] + v;  // resid + y, tn_add's operation; resid may be y
                 if (y_bf16)
-                    reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = bf16_from_f32(v);
+                    reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + n] = bf16_out(v);
                 else
                     reinterpret_cast<float*>(y)[(int64_t)m * N + n] = v;
             }

@@ -535,7 +535,7 @@ __global__ __launch_bounds__(QG_THREADS) void k_gemv_qk(const XT* __restrict__ x
                 const int64_t n = row0 + r;
                 if (bias) v = v + bias[n];
                 if (y_bf16)
-                    reinterpret_cast<uint16_t*>(y)[(int64_t)mr * N + n] = bf16_from_f32(v);
+                    reinterpret_cast<uint16_t*>(y)[(int64_t)mr * N + n] = bf16_out(v);
                 else
                     reinterpret_cast<float*>(y)[(int64_t)mr * N + n] = v;
             }
@@ -766,7 +766,7 @@ __global__ __launch_bounds__(QM_THREADS, 2) void k_gemm_qk(const uint16_t* __res
             float v = sumf[rt][r] + tot;
             if (bias) v = v + bv;
             if (y_bf16)
-                reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + col] = bf16_from_f32(v);
+                reinterpret_cast<uint16_t*>(y)[(int64_t)m * N + col] = bf16_out(v);
             else
                 reinterpret_cast<float*>(y)[(int64_t)m * N + col] = v;
         }

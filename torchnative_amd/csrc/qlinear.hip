@@ -736,7 +736,7 @@ __global__ __launch_bounds__(GEMV_THREADS) void k_gemv(const XT* __restrict__ x,
                 }
             }
             if (y_bf16)
-                reinterpret_cast<uint16_t*>(y)[(int64_t)mr * N + n] = bf16_from_f32(acc);
+                reinterpret_cast<uint16_t*>(y)[(int64_t)mr * N + n] = bf16_out(acc);
             else
                 reinterpret_cast<float*>(y)[(int64_t)mr * N + n] = acc;
         };
