@@ -212,11 +212,12 @@ struct FlashWork {
     uint32_t inl[FLASH_INLINE];  // the table itself when ncls <= FLASH_INLINE
 };
 
+// NQ: groups of 32 queries per workgroup (more than two: unsplit rows only).
 // MASK: 0 none; 1 an f32 additive mask; 2 one in the input format; 3 a bool
 // one (MaskRef), added to the scaled scores before the row maximum
 // (aten.rs:10383-10389)
-template <int D, int MASK = 0, bool F16 = false>
-__global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
+template <int D, int MASK = 0, bool F16 = false, int NQ = 2>
+__global__ __launch_bounds__(64 * NQ * FlashCfg<D>::KG) void k_flash16(
     const uint16_t* __restrict__ Qg, const uint16_t* __restrict__ Kg, const uint16_t* __restrict__ Vg, int Hq,
     int Hkv, int L, int S, float sl2, int causal, const FlashWork work, int nsplit, uint16_t* __restrict__ Og,
     float* __restrict__ lse, float* __restrict__ part_o, float2* __restrict__ part_ml, uint32_t* __restrict__ tickets,
@@ -224,7 +225,8 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     constexpr int KG = FlashCfg<D>::KG;        // key groups
     constexpr int BKW = FlashCfg<D>::BKW;      // keys per wave tile
     constexpr int NH = BKW / 32;               // 32-key halves per wave tile
-    constexpr int NW = 2 * KG;                 // waves
+    constexpr int BQ = 32 * NQ;                // queries per workgroup
+    constexpr int NW = NQ * KG;                // waves
     constexpr int NT = 64 * NW;                // threads
     constexpr int ROWS = KG * BKW;             // keys per ring stage
     constexpr int STAGE = ROWS * D;            // elements of one K (or V) stage
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     // landing in the other stage, and inserts no blanket vmcnt(0)
     __shared__ __align__(16) uint16_t sK0[STAGE], sK1[STAGE];
     __shared__ __align__(16) uint16_t sV0[STAGE], sV1[STAGE];
-    __shared__ float2 s_ml[KG / 2][2][64];
+    __shared__ float2 s_ml[KG / 2][NQ][64];
     __shared__ uint32_t s_ticket;
     auto stK = [&](auto sc) -> uint16_t* {
         if constexpr (decltype(sc)::value == 0) return sK0; else return sK1;
@@ -247,9 +249,9 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, kept in a scalar register
-    const int qw = w & 1, kg = w >> 1;                       // query half, key group
+    const int qw = w % NQ, kg = w / NQ;                      // query group, key group
     const int lq = lane & 31, hh = lane >> 5;
-    const int nqb = (L + F3_BQ - 1) / F3_BQ;
+    const int nqb = (L + BQ - 1) / BQ;
     const int cidx = (int)blockIdx.x / work.bh;
     const int bh = (int)blockIdx.x % work.bh;
     const uint32_t cl = work.ncls == 0              ? (uint32_t)(nqb - 1 - cidx)
@@ -258,10 +260,10 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     const int qt = (int)(cl & 0xffffu), split = (int)(cl >> 16);
     const int h = bh % Hq, b = bh / Hq;
     const int kvh = h / (Hq / Hkv);
-    const int q0 = qt * F3_BQ;
+    const int q0 = qt * BQ;
     const int qw0 = q0 + qw * 32;            // first query of this wave
     const int qi = qw0 + lq;
-    const int kend = causal ? min(S, q0 + F3_BQ) : S;
+    const int kend = causal ? min(S, q0 + BQ) : S;
     const int ntiles_row = (kend + F3_BK - 1) / F3_BK;
     const int nsplit_row = row_splits(ntiles_row, work.target);
     const int k_lo = split * ntiles_row / nsplit_row * F3_BK;         // this item's keys: [k_lo, k_hi)
@@ -313,8 +315,8 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     // The mask quads of a stage are requested with its K and V. (Loaded where
     // they are used, each wait for them also waited for the next stage's K and V,
     // requested just before: 2 x 16 heads, 1000 keys, D 128, f16, took 46 us with a
-    // key mask and 56 with a full one, against 35.5 without; now 39 and 41. 1001 keys,
-    // whose rows lie at any alignment, bf16: 109 with a full mask, now 34.)
+    // key mask and 56 with a full one, against 35.5 without; 39 and 41 since. 1001 keys,
+    // whose rows lie at any alignment, bf16: 109 with a full mask, 34 since.)
     using MA = MaskAhead<MASK == 0 ? 3 : MASK, F16>;
     [[maybe_unused]] const MA ma(mask, b, h, qi, L, S);
     [[maybe_unused]] typename MA::quad mq[2][4 * NH];
@@ -489,16 +491,16 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     // Tree merge of the key groups through LDS: in the round of width `half`,
     // group kg + half hands its (m, l, O) to group kg. Lane l of wave (qw, g)
     // holds the same (query, d) entries for every g. The O buffers of a round
-    // take 2*half wave slots of D*128 bytes, laid over the ring arrays (every
+    // take NQ*half wave slots of D*128 bytes, laid over the ring arrays (every
     // load has landed and been read once the first barrier has passed).
     constexpr int WSLOT = D / 32 * 16 * 64;        // floats per wave slot
     constexpr int PER_ARR = STAGE / 2 / WSLOT;     // wave slots per ring array
-    static_assert(PER_ARR >= 1 && KG <= 4 * PER_ARR, "merge slots must fit in the ring");
+    static_assert(PER_ARR >= 1 && KG / 2 * NQ <= 4 * PER_ARR, "merge slots must fit in the ring");
 #pragma unroll
     for (int half = KG / 2; half >= 1; half /= 2) {
         __syncthreads();
         if (kg >= half && kg < 2 * half) {
-            const int x = (kg - half) * 2 + qw;  // wave slot
+            const int x = (kg - half) * NQ + qw;  // wave slot
             float* arr = reinterpret_cast<float*>(x / PER_ARR == 0 ? sK0 : x / PER_ARR == 1 ? sK1
                                                   : x / PER_ARR == 2 ? sV0 : sV1);
             float* xo = arr + (x % PER_ARR) * WSLOT;
@@ -510,7 +512,7 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
         }
         __syncthreads();
         if (kg < half) {
-            const int x = kg * 2 + qw;
+            const int x = kg * NQ + qw;
             const float* arr = reinterpret_cast<const float*>(x / PER_ARR == 0 ? sK0 : x / PER_ARR == 1 ? sK1
                                                               : x / PER_ARR == 2 ? sV0 : sV1);
             const float* xo = arr + (x % PER_ARR) * WSLOT;
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(128 * FlashCfg<D>::KG) void k_flash16(
     const int64_t row = ((int64_t)b * Hq + h) * L + qi;
     if (nsplit_row > 1) {
         merge_split_rows<D, F16>(part_o, part_ml, tickets, nsplit, split, nsplit_row, (int64_t)bh * L + q0,
-                            min(F3_BQ, L - q0), bh * nqb + qt, kg == 0 && qi < L, qi - q0, hh, o, m, l, Og, lse,
+                            min(BQ, L - q0), bh * nqb + qt, kg == 0 && qi < L, qi - q0, hh, o, m, l, Og, lse,
                             s_ticket);
         return;
     }
@@ -1669,9 +1671,9 @@ __global__ __launch_bounds__(D) void k_decode_sk_combine(const float* __restrict
     for (int64_t w0 = w_lo + CB; w0 <= w_hi; w0 += CB) batch(w0);
     const float mu = (mm == -INFINITY) ? 0.0f : mm;
     if constexpr (std::is_same<OT, _Float16>::value)
-        reinterpret_cast<uint16_t*>(out)[((int64_t)b * Hq + h) * D + d] = f16_from_f32(acc / tl);
+        reinterpret_cast<uint16_t*>(out)[((int64_t)b * Hq + h) * D + d] = f16_out(acc / tl);
     else if constexpr (sizeof(OT) == 2)
-        out[((int64_t)b * Hq + h) * D + d] = bf16_from_f32(acc / tl);
+        out[((int64_t)b * Hq + h) * D + d] = bf16_out(acc / tl);
     else
         out[((int64_t)b * Hq + h) * D + d] = acc / tl;
     if (lse && d == 0) lse[(int64_t)b * Hq + h] = mu * LN2 + logf(tl);
@@ -1935,9 +1937,9 @@ __global__ __launch_bounds__(D) void k_decode_combine(const float* __restrict__ 
         acc = acc + part_o[(base + s) * D + d] * f;
     }
     if constexpr (std::is_same<OT, _Float16>::value)
-        reinterpret_cast<uint16_t*>(out)[((int64_t)b * Hq + h) * D + d] = f16_from_f32(acc / tl);
+        reinterpret_cast<uint16_t*>(out)[((int64_t)b * Hq + h) * D + d] = f16_out(acc / tl);
     else if constexpr (sizeof(OT) == 2)
-        out[((int64_t)b * Hq + h) * D + d] = bf16_from_f32(acc / tl);
+        out[((int64_t)b * Hq + h) * D + d] = bf16_out(acc / tl);
     else
         out[((int64_t)b * Hq + h) * D + d] = acc / tl;
     if (lse && d == 0) lse[(int64_t)b * Hq + h] = mu * LN2 + logf(tl);
@@ -2585,6 +2587,43 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
                                   static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
                                   static_cast<const uint16_t*>(v), B, Hq, Hkv, L, S, sl2, c,
                                   static_cast<uint16_t*>(out), lse);
+        auto qq = static_cast<const uint16_t*>(q);
+        auto kk = static_cast<const uint16_t*>(k);
+        auto vv = static_cast<const uint16_t*>(v);
+        auto oo = static_cast<uint16_t*>(out);
+        const bool h16 = dtype == TN_F16;
+        // Non-causal rows at head dim 128 whose 64-query blocks are more than the
+        // compute units, and their 128-query blocks are not: eight-wave workgroups,
+        // one a unit, unsplit. The list below gives such calls a second round, or
+        // splits their rows (bf16, us, list and here: 9 heads 2048 keys 55.3, 38.5;
+        // 16 heads 1664 keys 56, 34; 2 x 16 heads 1000 keys 27.0, 25.8). Fewer blocks
+        // leave units idle here (8 heads 2000 keys 35.2, 38.5), more come in coarse
+        // rounds (2 x 16 heads 1300 keys 51, 55), and causal rows leave the units of
+        // short ones idle (16 heads 1664 keys 27.2, 33.8).
+        int units = 0;
+        TN_TRY(resident_workgroups(reinterpret_cast<const void*>(&k_flash16<128, 0, false, 4>), 512, 0, &units));
+        const int64_t wide = B * Hq * cdiv(L, 128);
+        if (D == 128 && !c && wide <= units && B * Hq * cdiv(L, F3_BQ) > units) {
+            FlashWork work{};
+            work.target = INT32_MAX;
+            work.bh = (int)(B * Hq);
+#define TN_WIDE(MK, H)                                                                                               \
+    hipLaunchKernelGGL((k_flash16<128, MK, H, 4>), dim3((unsigned)wide), dim3(512), 0, st, qq, kk, vv, (int)Hq,   \
+                       (int)Hkv, (int)L, (int)S, sl2, c, work, 1, oo, lse, nullptr, nullptr, nullptr, mref, mahead)
+#define TN_WIDE_MK(H)                     \
+    do {                                  \
+        if (mk == 0) TN_WIDE(0, H);       \
+        else if (mk == 1) TN_WIDE(1, H);  \
+        else if (mk == 3) TN_WIDE(3, H);  \
+        else TN_WIDE(2, H);               \
+    } while (0)
+            if (h16) TN_WIDE_MK(true);
+            else TN_WIDE_MK(false);
+#undef TN_WIDE_MK
+#undef TN_WIDE
+            TN_LAUNCHED();
+            return TN_OK;
+        }
         // resident workgroups of the prefill kernel: the slots the schedule is planned over
         int slots = 0;
         tn_status sp = resident_workgroups(D == 64 ? reinterpret_cast<const void*>(&k_flash16<64>)
@@ -2615,10 +2654,6 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
             s = tickets(st, (size_t)(B * Hq) * (size_t)cdiv(L, F3_BQ), &tick);
             if (s != TN_OK) return s;
         }
-        auto qq = static_cast<const uint16_t*>(q);
-        auto kk = static_cast<const uint16_t*>(k);
-        auto vv = static_cast<const uint16_t*>(v);
-        auto oo = static_cast<uint16_t*>(out);
         // split rows are merged inside the kernel (merge_split_rows)
 #define TN_FLASH(DD, MK, H)                                                                                      \
     hipLaunchKernelGGL((k_flash16<DD, MK, H>), dim3((unsigned)nitems), dim3(128 * FlashCfg<DD>::KG), 0, st, qq, kk, \
@@ -2631,7 +2666,6 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
         else if (mk == 3) TN_FLASH(DD, 3, H); \
         else TN_FLASH(DD, 2, H);        \
     } while (0)
-        const bool h16 = dtype == TN_F16;
         if (D == 64) {
             if (h16) TN_FLASH_MK(64, true); else TN_FLASH_MK(64, false);
         } else {
