@@ -60,3 +60,22 @@ def test_the_librarys_assembly_reads_no_mfma_result_early():
     results = H.scan_sources()
     bad = [(src, f) for src, found in results.items() for f in found]
     assert not bad, "\n".join(f"{src}: {f[0][:60]}: {f[2]} after {f[3]} wait states" for src, f in bad[:20])
+
+
+def test_a_barrier_behind_an_unreturned_lds_read_is_found():
+    read, drain = "ds_read_b128 v[0:3], v9", "s_waitcnt vmcnt(0) lgkmcnt(0)"
+    assert len(H.open_barriers(_fn(read, "s_waitcnt vmcnt(0)", "s_barrier"), "test")) == 1
+    assert len(H.open_barriers(_fn(drain, ".LBB0_2:", "s_waitcnt vmcnt(0)", "s_barrier"), "test")) == 1  # a back edge
+    assert len(H.open_barriers(_fn(drain, read, "s_barrier"), "test")) == 1
+    assert H.open_barriers(_fn(read, drain, "s_barrier"), "test") == []
+
+
+@pytest.mark.skipif(shutil.which(H.build.HIPCC) is None and not __import__("os").path.exists(H.build.HIPCC),
+                    reason="hipcc is not installed")
+@pytest.mark.parametrize("src,kernel", [("flash_any.hip", "k_flash_any"), ("qgemm.hip", "k_qgemm"),
+                                        ("dense.hip", "k_dense_lds")])
+def test_ring_stages_are_read_before_they_are_opened(tmp_path, src, kernel):
+    """The kernels whose LDS rings are filled by loads in assembly."""
+    asm = H.assembly(src, str(tmp_path))
+    assert kernel in asm
+    assert H.open_barriers(asm, kernel) == []

@@ -165,7 +165,8 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
                 mcur[rq] = mq[rq];
             }
         }
-        asm volatile("" ::: "memory");
+        // this wave's reads of the other stage, which the barrier opens to issue()
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (st + 1 < st_hi) {

@@ -15,6 +15,13 @@ is active (the fall-through of `s_cbranch_execnz`, the target of
 `s_cbranch_execz`) vector instructions read nothing until a scalar
 instruction writes `exec` again.
 
+A second check (`open_barriers`) is for kernels that fill a ring in LDS with
+loads the compiler does not see (LdsDma, attn_common.h): a barrier opens a
+stage to the next loads, so the reads of it must have returned, and no
+dependence makes the compiler wait for them. It reports every `s_barrier`
+behind a wait for such loads (`vmcnt`) that has no `s_waitcnt lgkmcnt(0)` since
+the last LDS access or label.
+
 `python -m torchnative_amd.hazard_scan` compiles every source to assembly
 with the build's flags and prints the findings; tests/test_hazard_scan.py
 requires there to be none.
@@ -112,12 +119,38 @@ def scan_function(lines, name="?", max_depth=4):
     return found
 
 
-def scan_text(asm: str):
+def _functions(asm: str):
+    """[(name, lines)] of an assembly text."""
     lines = asm.split("\n")
     starts = [k for k, l in enumerate(lines) if _FUNC.match(l)]
+    return [(_FUNC.match(lines[a]).group(1), lines[a + 1:b]) for a, b in zip(starts, starts[1:] + [len(lines)])]
+
+
+def scan_text(asm: str):
+    return [f for name, lines in _functions(asm) for f in scan_function(lines, name)]
+
+
+def open_barriers(asm: str, kernel: str):
+    """[(function, index)] of the barriers in functions named `kernel` that open
+    a ring stage with LDS accesses that may be outstanding."""
     found = []
-    for a, b in zip(starts, starts[1:] + [len(lines)]):
-        found += scan_function(lines[a + 1:b], _FUNC.match(lines[a]).group(1))
+    for name, lines in _functions(asm):
+        if kernel not in name:
+            continue
+        ins, labels = _parse(lines)
+        targets, drained, ring = set(labels.values()), False, False
+        for i, (op, args, text) in enumerate(ins):
+            if i in targets:
+                drained = ring = False
+            if op.startswith("ds_"):
+                drained = False
+            if op == "s_waitcnt":
+                drained = drained or "lgkmcnt(0)" in text
+                ring = ring or "vmcnt" in text
+            if op == "s_barrier":
+                if ring and not drained:
+                    found.append((name, i))
+                ring = False
     return found
 
 
