@@ -158,6 +158,47 @@ def test_decode(tn, dtype, Hq, Hkv, D, lens, cap):
                  vw[b:b + 1, :, :n])
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("shape,causal,scale", [
+    # B, Hq, Hkv, L, S, D: rows and key groups, split keys, the decode entry (L 1), a negative scale
+    ((1, 2, 2, 70, 200, 96), False, None), ((2, 2, 1, 90, 90, 72), True, None), ((1, 1, 1, 33, 40, 256), False, None),
+    ((1, 2, 1, 5, 2100, 80), False, None), ((2, 8, 2, 1, 1500, 96), False, None), ((1, 2, 2, 40, 70, 64), False, -0.2)])
+def test_infinite_values(tn, shape, causal, scale, dtype):
+    """V infinite in single keys of some columns: every row that gives the key
+    a probability gets that infinity, both signs in a column NaN, as f32
+    probabilities do, however small the probability (about 1e-28 here); the other
+    columns keep their bits."""
+    B, Hq, Hkv, L, S, D = shape
+    rng = np.random.default_rng(S)
+    q, k, v = (rng.standard_normal(s) for s in ((B, Hq, L, D), (B, Hkv, S, D), (B, Hkv, S, D)))
+    # key 0 far below the other keys: a score of -64 (-51 with the negative scale)
+    q[..., 0], k[:, :, 1:, 0] = 32.0, 0.0
+    k[:, :, 0, 0] = -2.0 * np.sqrt(D) if scale is None else 8.0
+    inf = v.copy()
+    inf[:, :, 0, 3], inf[:, :, 0, 5], inf[:, :, min(S - 1, 37) if not causal else 0, 7] = np.inf, -np.inf, np.inf
+    if not causal:
+        inf[:, :, S // 2, 9], inf[:, :, S // 2 + 1, 9] = np.inf, -np.inf
+    cols = [3, 5, 7] + ([] if causal else [9])
+    qd, kd = _dev(tn, dtype, q), _dev(tn, dtype, k)
+    outs = []
+    for val in (inf, v):
+        vd = _dev(tn, dtype, val)
+        if L == 1:
+            ln = tn.tensor(np.full(B, S, np.int32), device="hip")
+            o, _ = tn.sdpa_decode(_dev(tn, dtype, q[:, :, 0]), kd, vd, ln, S)
+            outs.append(o.numpy().reshape(B, Hq, 1, D))
+        else:
+            o, _ = tn._aten_dispatch(OP, qd, kd, vd, 0.0, causal, scale=scale)
+            outs.append(o.numpy())
+    rest = [c for c in range(D) if c not in cols]
+    assert np.isfinite(outs[1]).all() and np.array_equal(outs[0][..., rest], outs[1][..., rest])
+    with np.errstate(invalid="ignore"):
+        want = O.sdpa(*(t.numpy().astype(np.float64) for t in (qd, kd)), _dev(tn, dtype, inf).numpy().astype(np.float64),
+                      is_causal=causal, scale=scale, threads=16)[0]
+    assert np.array_equal(outs[0][..., cols], want[..., cols].astype(outs[0].dtype), equal_nan=True)
+    assert np.isposinf(want[..., 3]).all() and np.isneginf(want[..., 5]).all()
+
+
 def test_captured_without_a_workspace_runs_unsplit(tn):
     """A call that would split its keys, captured on a stream that holds no
     workspace (nothing may be allocated then): it runs unsplit, three replays

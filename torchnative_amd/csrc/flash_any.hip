@@ -63,6 +63,29 @@ constexpr float P_BIAS = F16 ? 6.0f : 0.0f;
 template <bool F16>
 constexpr float P_UNIT = F16 ? 1.0f / 64 : 1.0f;  // takes the factor out of the sum again, exactly
 
+// P = hi + lo must give P * V's infinity where V holds one. hi carries the sign
+// of P and is positive wherever P is: an f16 hi would round to zero under 2^-25
+// (x times 2^126 is x, or past the smallest f16, or zero). lo has either sign and
+// is zero where hi is exact, so it multiplies V clamped to the largest finite
+// value (a NaN too: hi's product keeps it).
+template <bool F16>
+__device__ __attribute__((always_inline)) inline float hi_of(float x) {
+    if constexpr (F16) return __builtin_amdgcn_fmed3f(x, x * 0x1p126f, 0x1p-24f);
+    else return x;
+}
+
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+// As signed numbers only positive patterns lie past +max, as unsigned ones only
+// negative patterns past -max.
+template <bool F16>
+__device__ __attribute__((always_inline)) inline uint32_t finite2(uint32_t w) {
+    constexpr short TOP = F16 ? 0x7bff : 0x7f7f;
+    constexpr unsigned short LOW = F16 ? 0xfbff : 0xff7f;
+    const s16x2 a = __builtin_elementwise_min(__builtin_bit_cast(s16x2, w), (s16x2){TOP, TOP});
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), (u16x2){LOW, LOW}));
+}
+
 template <int DT, int NQ, bool MASKED, bool F16>
 __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArgs a) {
     using C = AnyCfg<DT, NQ>;
@@ -246,7 +269,7 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float x0 = p[8 * j + 2 * e], x1 = p[8 * j + 2 * e + 1];
-                hi[e] = E::pack_p(x0, x1);
+                hi[e] = E::pack_p(hi_of<F16>(x0), hi_of<F16>(x1));
                 lo[e] = E::pack_p(x0 - E::lo(hi[e]), x1 - E::hi(hi[e]));
             }
             ph[j] = __builtin_bit_cast(V8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
@@ -263,8 +286,10 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
                 const uint2 lo = lds_read_tr16(tV + r0 * P + swz(r0, col >> 3) * 8 + (col & 7));
                 const uint2 hi = lds_read_tr16(tV + r1 * P + swz(r1, col >> 3) * 8 + (col & 7));
                 const V8 va = __builtin_bit_cast(V8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                const V8 vf = __builtin_bit_cast(V8, make_uint4(finite2<F16>(lo.x), finite2<F16>(lo.y),
+                                                                finite2<F16>(hi.x), finite2<F16>(hi.y)));
                 o[dt] = E::mfma(va, ph[j], o[dt]);
-                o[dt] = E::mfma(va, pl[j], o[dt]);
+                o[dt] = E::mfma(vf, pl[j], o[dt]);
             }
         }
     }
