@@ -87,8 +87,7 @@ def test_scales_across_every_f16_regime(tn, fmt):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 def test_operands_at_any_element(tn, fmt):
-    """bf16 and f32 rows one element past an aligned address, and a code plane
-    that is not 16-byte aligned (it runs on the GEMV)."""
+    """bf16 and f32 rows one element past an aligned address."""
     from torchnative_amd import _lib
 
     rng = np.random.default_rng(5)
@@ -102,12 +101,29 @@ def test_operands_at_any_element(tn, fmt):
         y = tn.empty((m, n), "float32", "hip")
         _lib.check(fn(None, buf.data_ptr() + es, code, m, k, *q._planes(), n, None, y.data_ptr(), _lib.TN_F32))
         assert y.numpy().tobytes() == _linear(fmt)(x, blob, n, threads=8).tobytes(), dt
-    x = tn.tensor(rng.standard_normal((m, k)).astype(np.float32), device="hip")
-    moved = tn.tensor(np.concatenate([np.zeros(8, np.uint8), q._qs.numpy()]), device="hip")
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("m,n,k,off,xoff", [
+    # both tile shapes of such a plane (up to 6144 tiles, and more), stages in rings of 4 and 3: one block, less than
+    # a ring, remainders; one to four rows with an unaligned x; a row past the GEMV's limits
+    (21, 50, 320, 8, 0), (7, 33, 32, 1, 1), (64, 70, 544, 4, 0), (5, 40, 128, 2, 0), (130, 11000, 160, 8, 1),
+    (400, 4000, 416, 3, 0), (1, 40, 320, 8, 1), (4, 33, 64, 1, 1), (2, 5, 40960, 12, 0)])
+def test_code_plane_at_any_byte(tn, fmt, m, n, k, off, xoff):
+    from torchnative_amd import _lib
+
+    rng = np.random.default_rng(m + n + off)
+    blob = _blob(fmt, n, k, 6)
+    q = tn._quantized_from_blob(blob, (n, k), fmt, device="hip")
+    buf = tn.tensor(rng.standard_normal(m * k + xoff).astype(np.float32), device="hip")
+    codes = q._qs.numpy().view(np.uint8).reshape(-1)
+    moved = tn.tensor(np.concatenate([np.full(off, 0x5A, np.uint8), codes, np.full(16 - off, 0xA5, np.uint8)]), device="hip")
     y = tn.empty((m, n), "float32", "hip")
-    _lib.check(fn(None, x.data_ptr(), _lib.TN_F32, m, k, moved.data_ptr() + 8, q._d.data_ptr(), n, None, y.data_ptr(),
-                  _lib.TN_F32))
-    assert y.numpy().tobytes() == _linear(fmt)(x.numpy(), blob, n, threads=8).tobytes()
+    _lib.check(getattr(_lib.lib(), f"tn_{fmt}_linear")(None, buf.data_ptr() + 4 * xoff, _lib.TN_F32, m, k,
+                                                      moved.data_ptr() + off, q._d.data_ptr(), n, None, y.data_ptr(),
+                                                      _lib.TN_F32))
+    want = _linear(fmt)(buf.numpy()[xoff:].reshape(m, k), blob, n, threads=16)
+    assert y.numpy().tobytes() == want.tobytes()
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])

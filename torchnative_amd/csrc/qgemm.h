@@ -11,7 +11,7 @@ struct QGemmArgs {
     int x_bf16;
     int64_t m, k;
     int xm, hd;
-    const uint8_t* qs;  // 16-byte aligned
+    const uint8_t* qs;  // any alignment (16-byte aligned ones are read straight into LDS)
     const uint16_t* d;
     int64_t n;
     const float* bias;

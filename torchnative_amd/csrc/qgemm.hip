@@ -22,7 +22,8 @@
 //   prepass writes the activation codes in that order, tile by tile, so that a
 //   product's operand is 512 consecutive bytes.
 // - A ring of NS stages of KB blocks in LDS, filled by loads that go straight
-//   to LDS; one barrier per stage. Within a stage block t + 2 is read from LDS,
+//   to LDS (a code plane that is not 16-byte aligned through registers, a stage
+//   later: DMA false); one barrier per stage. Within a stage block t + 2 is read from LDS,
 //   block t + 1's products are issued and block t's roundings done, in that
 //   order, so that neither LDS nor the matrix core is waited for.
 //
@@ -94,14 +95,14 @@ struct QGeo {
     static constexpr int OW = 0, OA = OW + IW * 1024, OX = OA + IA * 1024, OD = OX + IX * 1024, STAGE = OD + ID * 256;
 };
 
-template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS>
+template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS, bool DMA>
 __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf, const float* __restrict__ dxf, int M,
                                                  int mtiles, int nb, const uint8_t* __restrict__ qs,
                                                  const uint16_t* __restrict__ dw, int N, const float* __restrict__ bias,
                                                  void* y, int y_bf16, const float* resid) {
     using G = QGeo<FMT, RT, CT, WM, WN, KB, NS>;
     constexpr int CB = G::CB, BN = G::BN, AHEAD = RT * CT < 4 ? 2 : 1;
-    constexpr int PER_STAGE = G::LW + G::LA + G::LX + G::LD;
+    constexpr int PER_STAGE = (DMA ? G::LW : 0) + G::LA + G::LX + G::LD;
     static_assert((NS - 2) * PER_STAGE < 64, "loads in flight");
     // the ring, then 1 KB that takes the zeros of a wave with no load left to issue
     __shared__ __align__(16) uint8_t ring[NS * G::STAGE + 1024];
@@ -147,12 +148,36 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
         const int p = (4 * i + wave) * 64 + lane, b = p / (4 * BN) * 4 + (p & 3), c = p % (4 * BN) / 4;
         vd[i] = b < KB ? (uint32_t)(c * nb + b) * 2u : BUF_OOB;
     }
+    // the codes of the last issued stage on their way through registers, and its slot
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    [[maybe_unused]] u32x4 pend[G::LW];
+    [[maybe_unused]] int pslot = 0;
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (!DMA) {
+#pragma unroll
+            for (int i = 0; i < G::LW; i++)
+                if (4 * i + wave < G::IW)
+                    *reinterpret_cast<u32x4*>(ring + pslot * G::STAGE + G::OW + (4 * i + wave) * 1024 + lane * 16) = pend[i];
+        }
+    };
     auto issue = [&](int st, int slot) __attribute__((always_inline)) {
         uint8_t* const s = ring + slot * G::STAGE;
         uint8_t* const spare = ring + NS * G::STAGE;
+        if constexpr (DMA) {
 #pragma unroll
-        for (int i = 0; i < G::LW; i++)
-            rw.load16(vw[i] + (uint32_t)(st * KB * CB), 4 * i + wave < G::IW ? s + G::OW + (4 * i + wave) * 1024 : spare);
+            for (int i = 0; i < G::LW; i++)
+                rw.load16(vw[i] + (uint32_t)(st * KB * CB), 4 * i + wave < G::IW ? s + G::OW + (4 * i + wave) * 1024 : spare);
+        } else {
+            typedef u32x4 anywhere __attribute__((aligned(1)));
+            const uint32_t bytes = (uint32_t)(ncols * nb * CB);
+#pragma unroll
+            for (int i = 0; i < G::LW; i++) {
+                // (past the end: the first codes again, unused)
+                const uint32_t o = vw[i] + (uint32_t)(st * KB * CB);
+                pend[i] = *reinterpret_cast<const anywhere*>(qs + (int64_t)n0 * nb * CB + (o < bytes ? o : 0u));
+            }
+            pslot = slot;
+        }
 #pragma unroll
         for (int i = 0; i < G::LA; i++)
             ra.load16(va[i] + (uint32_t)(st * KB * 512), 4 * i + wave < G::IA ? s + G::OA + (4 * i + wave) * 1024 : spare);
@@ -191,7 +216,6 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
         }
     };
     // the weight scales of four blocks at once (the dword's low half)
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     struct Scales {
         u32x4 d[CT];
     };
@@ -244,13 +268,17 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    for (int st = 0; st < min(NS - 1, nst); st++) issue(st, st);
+    for (int st = 0; st < min(NS - 1, nst); st++) {
+        if (st > 0) flush();
+        issue(st, st);
+    }
     // Registers of block t: blk[t mod 2 AHEAD], products sv[t mod AHEAD]. Few
     // tiles: block t + 2 is read and t + 1's products issued ahead of t's
     // roundings. Four and more hide a product's latency by themselves: one
     // block ahead, half the registers.
     Block blk[2 * AHEAD];
     i32x4 sv[AHEAD][RT][CT];
+    flush();
     landed(0);
     if (NS - 1 < nst) issue(NS - 1, NS - 1);
     lread(ring, 0, blk[0]);
@@ -273,7 +301,9 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
             if (!WHOLE && b >= left) break;
             if (WHOLE && b == KB - AHEAD) {
                 // every read of this stage has been issued: its slot takes
-                // stage st + NS once all waves are here
+                // stage st + NS once all waves are here (and stage st - 1's
+                // slot, free since the barrier before, the codes issued there)
+                if (st + NS - 1 < nst) flush();
                 landed(st + 1);
                 if (st + NS < nst) issue(st + NS, slot);
             }
@@ -315,11 +345,11 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
     }
 }
 
-template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS>
+template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS, bool DMA = true>
 void launch(hipStream_t st, const QGemmArgs& a, const uint8_t* xf, const float* dxf, int mt, int nb) {
     using G = QGeo<FMT, RT, CT, WM, WN, KB, NS>;
     const dim3 grid((unsigned)(cdiv(mt, G::RTT) * cdiv(a.n, G::BN)));
-    hipLaunchKernelGGL((k_qgemm<FMT, RT, CT, WM, WN, KB, NS>), grid, dim3(QG_TH), 0, st, xf, dxf, (int)a.m, mt, nb,
+    hipLaunchKernelGGL((k_qgemm<FMT, RT, CT, WM, WN, KB, NS, DMA>), grid, dim3(QG_TH), 0, st, xf, dxf, (int)a.m, mt, nb,
                        a.qs, a.d, (int)a.n, a.bias, a.y, a.y_bf16, a.resid);
 }
 
@@ -341,6 +371,14 @@ void launch(hipStream_t st, const QGemmArgs& a, const uint8_t* xf, const float* 
 template <int FMT>
 void launch_fmt(hipStream_t st, const QGemmArgs& a, const uint8_t* xf, const float* dxf, int mt, int nb) {
     const int64_t tiles = mt * cdiv(a.n, 16);
+    // a code plane off 16 bytes: loads straight to LDS need whole granules ([m, 4096]
+    // x [14336, 4096] q4_0, m 16, 128, 512, us: 24.4, 44.9, 126.4; aligned 17.9,
+    // 44.5, 123.0)
+    if (reinterpret_cast<uintptr_t>(a.qs) % 16 != 0) {
+        if (tiles <= 6144) launch<FMT, 1, 1, 2, 2, 4, 4, false>(st, a, xf, dxf, mt, nb);
+        else launch<FMT, 2, 2, 2, 2, 4, 3, false>(st, a, xf, dxf, mt, nb);
+        return;
+    }
     if (mt == 1) launch<FMT, 1, 1, 1, 4, 8, FMT == FMT_Q8_0 ? 3 : 4>(st, a, xf, dxf, mt, nb);
     else if (tiles <= 2560) launch<FMT, 1, 1, 2, 2, 8, 3>(st, a, xf, dxf, mt, nb);
     else if (tiles <= 6144) launch<FMT, 1, 1, 2, 2, 4, 4>(st, a, xf, dxf, mt, nb);
@@ -353,8 +391,6 @@ tn_status qgemm_launch(hipStream_t st, const QGemmArgs& a) {
     // row and tile counts as int, a workgroup's operands under 2^31 bytes
     if (a.m > INT32_MAX - 15 || a.n > INT32_MAX || a.k > INT32_MAX || 4 * (a.k / QK) * 512 > INT32_MAX)
         return fail(TN_EVALUE, "torch._C._quantized_linear: shape too large");
-    if (reinterpret_cast<uintptr_t>(a.qs) % 16 != 0)
-        return fail(TN_EINVAL, "torch._C._quantized_linear: the weight's code plane must be 16-byte aligned");
     const int nb = (int)(a.k / QK);
     const int mt = (int)cdiv(a.m, 16);
     const int64_t blocks = (int64_t)mt * 16 * nb;

@@ -870,9 +870,8 @@ tn_status linear_impl(hipStream_t st, const XT* x, int64_t m, int64_t k, const u
         TN_TRY(workspace_or_none(st, qgemm_workspace(rows), &ws));
         if (ws) return qgemm_launch(st, rows);
     }
-    // the GEMV reads x in 16-byte pieces; an unaligned x takes the GEMM, whose
-    // direct loads in turn need the code plane aligned
-    if ((m <= GEMV_MAX_M || reinterpret_cast<uintptr_t>(qs) % 16 != 0) && nb <= GEMV_THREADS * Fmt<FMT>::GEMV_ITEMS && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+    // the GEMV reads x in 16-byte pieces; an unaligned x takes the GEMM
+    if (m <= GEMV_MAX_M && nb <= GEMV_THREADS * Fmt<FMT>::GEMV_ITEMS && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         // decode: GEMV in chunks of up to 4 rows of x (a row's result does not
         // depend on the chunking: every output is the same recurrence)
         int64_t r = 0;
