@@ -260,9 +260,13 @@ tn_status tn_dense_linear(void* stream, const float* x, int64_t m, int64_t k, co
  * Head dims 64 and 128 with scale > 0 run on MFMA kernels; so do 16-bit inputs
  * at any other multiple of 8 up to 256, or with another scale (the
  * probabilities as a sum of two 16-bit parts there), and f32 ones at any
- * multiple of 4 (unless a capture could not grow the stream's buffers). What is
- * left, and rows that are not 16-byte aligned, runs on a plain f32 kernel (f32
- * probabilities); a head dim past 256 is refused by name. */
+ * multiple of 4. What is left, and rows that are not 16-byte aligned, runs on a
+ * plain f32 kernel (f32 probabilities); a head dim past 256 is refused by name.
+ * Under capture, a call at head dims 64 or 128 whose stream holds too small a
+ * workspace is refused by name; at the others it runs without one: 16-bit
+ * inputs with the same bits, f32 ones on the plain kernel. The recorded graph
+ * keeps that slower form (4 heads, 1024 causal keys, f32, head dim 96: 518 us
+ * against 58); one such call on the stream before the capture avoids it. */
 tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, const void* v,
                       int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t S, int64_t D,
                       const void* attn_mask, int mask_dtype, const int64_t* mask_strides,
@@ -282,10 +286,13 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
  *   lse nullable f32 [B, Hq].
  * Head dims 64 and 128: split-KV with a combine pass, the partials in the
  * library workspace; so do 16-bit caches at any other multiple of 8 and f32
- * ones at any other multiple of 4 up to 256 (unsplit where a capture could not
- * grow the workspace); otherwise a head dim up to 256 runs on the plain kernel
- * (one workgroup per (sequence, head)). A sequence of length 0 gives NaN out
- * and -inf lse. */
+ * ones at any other multiple of 4 up to 256. There a capture that could not
+ * grow the workspace is not refused: one workgroup takes the splits of its
+ * rows in turn, the same bits but slower (24 heads of 12000 bf16 keys at head
+ * dim 96: 146 us against 37), and so does every replay of that graph; one such
+ * call on the stream before the capture avoids it. Otherwise a head dim up to
+ * 256 runs on the plain kernel (one workgroup per (sequence, head)). A sequence
+ * of length 0 gives NaN out and -inf lse. */
 tn_status tn_sdpa_decode(void* stream, int dtype, const void* q, const void* k_cache,
                          const void* v_cache, int64_t B, int64_t Hq, int64_t Hkv, int64_t cap,
                          int64_t D, const int32_t* lens, int64_t max_len, double scale,
@@ -301,7 +308,10 @@ tn_status tn_sdpa_decode(void* stream, int dtype, const void* q, const void* k_c
  * work buffer would exceed the array refuses with TN_EVALUE naming both
  * sizes (e.g. config 4's B=16, 32/8 heads, head dim 128 needs about 4.5 MB).
  * Every call on a GPU shares that GPU's array: calls that overlap on one GPU
- * (on different streams) race, so serialise them. */
+ * (on different streams) race, so serialise them. Head dims other than 64 and
+ * 128 do not use the array: such a call splits its keys if its stream is not
+ * under capture and already holds a large enough workspace (from an earlier
+ * call of another entry), else it takes the splits in turn, as above. */
 #define TN_DECODE_SCRATCH_BYTES (8u << 20)
 tn_status tn_sdpa_decode_noalloc(void* stream, int dtype, const void* q, const void* k_cache,
                                  const void* v_cache, int64_t B, int64_t Hq, int64_t Hkv, int64_t cap,

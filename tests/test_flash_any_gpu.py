@@ -199,32 +199,53 @@ def test_infinite_values(tn, shape, causal, scale, dtype):
     assert np.isposinf(want[..., 3]).all() and np.isneginf(want[..., 5]).all()
 
 
-def test_captured_without_a_workspace_runs_unsplit(tn):
-    """A call that would split its keys, captured on a stream that holds no
-    workspace (nothing may be allocated then): it runs unsplit, three replays
-    on changing inputs within the bound."""
+@pytest.mark.parametrize("dtype,shape,causal,scale,masked", [
+    # every padded width, one and two row halves; a mask; causal splits without a key; 64 and 128 by the scale's sign
+    ("bfloat16", (1, 2, 1, 5, 2100, 96), False, None, False), ("float16", (1, 2, 1, 40, 1100, 32), False, None, True),
+    ("float16", (1, 1, 1, 70, 1500, 128), False, -0.1, True), ("bfloat16", (1, 2, 2, 600, 600, 80), True, None, False),
+    ("bfloat16", (2, 1, 1, 7, 900, 64), False, -0.2, False), ("bfloat16", (1, 1, 1, 30, 800, 256), False, None, True),
+    ("float16", (1, 2, 2, 33, 513, 200), False, None, False)])
+def test_captured_without_a_workspace_gives_the_same_bits(tn, dtype, shape, causal, scale, masked):
+    """A call that splits its keys, captured on a stream that holds no
+    workspace (nothing may be allocated then): one workgroup takes its rows'
+    splits in turn; three replays on changing inputs, the eager call's bits
+    and within the bound."""
     from torchnative_amd import _lib as L
 
     f = L.lib()
-    shape = (1, 2, 1, 5, 2100, 96)
     B, Hq, Hkv, Lq, S, D = shape
-    (q, k, v), _ = _inputs(tn, "bfloat16", *shape, seed=3)
-    out, lse = tn.empty((B, Hq, Lq, D), "bfloat16", "hip"), tn.empty((B, Hq, Lq), "float32", "hip")
+    code, sc = (L.TN_BF16 if dtype == "bfloat16" else L.TN_F16), float("nan") if scale is None else scale
+    (q, k, v), _ = _inputs(tn, dtype, *shape, seed=3)
+    add = np.random.default_rng(4).standard_normal((Lq, S)) if masked else None
+    md = _dev(tn, "float32", add) if masked else None
+    strides = (ctypes.c_int64 * 4)(0, 0, S, 1)
+    outs = [(tn.empty((B, Hq, Lq, D), dtype, "hip"), tn.empty((B, Hq, Lq), "float32", "hip")) for _ in range(2)]
+
+    def call(stream, out, lse):
+        L.check(f.tn_sdpa_fwd(stream, code, q.data_ptr(), k.data_ptr(), v.data_ptr(), B, Hq, Hkv, Lq, S, D,
+                              md.data_ptr() if masked else None, L.TN_F32 if masked else 0, strides if masked else None,
+                              int(causal), sc, out.data_ptr(), lse.data_ptr()))
+
     s = ctypes.c_void_p()
     L.check(f.tn_stream_create(ctypes.byref(s)))
     try:
         L.check(f.tn_stream_begin_capture(s))
-        L.check(f.tn_sdpa_fwd(s, L.TN_BF16, q.data_ptr(), k.data_ptr(), v.data_ptr(), B, Hq, Hkv, Lq, S, D, None, 0, None,
-                              0, float("nan"), out.data_ptr(), lse.data_ptr()))
+        call(s, *outs[0])
         g = ctypes.c_void_p()
         L.check(f.tn_stream_end_capture(s, ctypes.byref(g)))
         for i in range(3):
-            (q2, k2, v2), w = _inputs(tn, "bfloat16", *shape, seed=20 + i)
+            (q2, k2, v2), w = _inputs(tn, dtype, *shape, seed=20 + i)
             for a, b in ((q, q2), (k, k2), (v, v2)):
                 L.check(f.tn_memcpy_d2d(a.data_ptr(), b.data_ptr(), a.nbytes, s))
             L.check(f.tn_graph_launch(s, g))
             L.check(f.tn_stream_synchronize(s))
-            _compare("bfloat16", out.numpy().astype(np.float64), lse.numpy(), *w)
+            call(None, *outs[1])
+            tn.synchronize()
+            (o, lse), (o2, l2) = outs
+            assert o.bits().tobytes() == o2.bits().tobytes() and lse.numpy().tobytes() == l2.numpy().tobytes()
+            mask = None if md is None else np.ascontiguousarray(
+                np.broadcast_to(md.numpy().astype(np.float64), (B, Hq, Lq, S)))
+            _compare(dtype, o.numpy().astype(np.float64), lse.numpy(), *w, causal=causal, mask=mask, scale=scale)
         L.check(f.tn_graph_destroy(g))
     finally:
         L.check(f.tn_stream_destroy(s))

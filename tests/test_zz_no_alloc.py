@@ -4,9 +4,9 @@ fixed device array, for callers that cannot allocate.
 Checked against tn_sdpa_decode, which shares its kernels, bit for bit, on
 two calls in a row (the second smaller, so stale contents of the array from
 the first must not leak into it), on the stream-K path (bf16 and f16 caches),
-the split path of f32 caches, and a path that needs no buffer; the library's
-workspace counter shows the no-alloc calls allocate nothing; a call whose
-buffer would not fit the array is refused by name.
+the split path of f32 caches, and at the head dims other than 64 and 128, which
+do not use the array; the library's workspace counter shows the no-alloc calls
+allocate nothing; a call whose buffer would not fit the array is refused by name.
 """
 
 import ctypes
@@ -70,14 +70,54 @@ def test_noalloc_equals_the_allocating_entry_on_two_calls_in_a_row(tn, dtype):
         L.check(f.tn_stream_destroy(s.value))
 
 
-def test_noalloc_on_a_path_without_a_work_buffer(tn):
-    """Head dim 80 runs the plain kernel, which needs no buffer."""
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,D,cap,lens", [
+    ("bfloat16", 2, 4, 2, 80, 100, [100, 33]),  # too few keys to split
+    ("bfloat16", 3, 24, 24, 96, 3000, [3000, 0, 517]), ("float16", 1, 8, 1, 256, 2100, [2050]),
+    ("float16", 2, 40, 1, 32, 1500, [1, 1500]), ("float32", 1, 8, 8, 96, 3900, [3900]),
+    ("float32", 3, 6, 2, 40, 900, [900, 0, 65]), ("float32", 2, 10, 2, 256, 700, [700, 699]),
+    ("float32", 1, 4, 2, 20, 2000, [1999])])
+def test_other_head_dims_have_one_result(tn, dtype, B, Hq, Hkv, D, cap, lens):
+    """Both entries, eager and captured, on a stream that holds a workspace and
+    on one that holds none (where a workgroup takes its rows' splits in turn):
+    the same bits. The no-alloc entry allocates nothing."""
     from torchnative_amd import _lib as L
 
-    c = _case(tn, "bfloat16", 2, 4, 2, 80, 100, [100, 33], 15)
-    got = _run(tn, L.lib().tn_sdpa_decode_noalloc, c, None)
-    want = _run(tn, L.lib().tn_sdpa_decode, c, None)
-    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    f = L.lib()
+    c = _case(tn, dtype, B, Hq, Hkv, D, cap, lens, 15)
+    want = _run(tn, f.tn_sdpa_decode, c, None)
+
+    def same(got):
+        return all(g.tobytes() == w.tobytes() for g, w in zip(got, want))
+
+    code = {"bfloat16": L.TN_BF16, "float16": L.TN_F16, "float32": L.TN_F32}[dtype]
+    held = ctypes.c_void_p()
+    L.check(f.tn_stream_create(ctypes.byref(held)))
+    assert same(_run(tn, f.tn_sdpa_decode, c, held.value))
+    before = tn._hip_counters()["workspace_bytes"]
+    assert same(_run(tn, f.tn_sdpa_decode_noalloc, c, held.value))
+    bare = ctypes.c_void_p()
+    L.check(f.tn_stream_create(ctypes.byref(bare)))
+    try:
+        assert same(_run(tn, f.tn_sdpa_decode_noalloc, c, bare.value))
+        for stream in (bare, held):
+            for fn in (f.tn_sdpa_decode, f.tn_sdpa_decode_noalloc):
+                out, lse = tn.empty((B, Hq, D), dtype, "hip"), tn.empty((B, Hq), "float32", "hip")
+                L.check(f.tn_stream_begin_capture(stream))
+                L.check(fn(stream, code, c["q"].data_ptr(), c["k"].data_ptr(), c["v"].data_ptr(), B, Hq, Hkv, cap, D,
+                           c["lens"].data_ptr(), c["max_len"], float("nan"), out.data_ptr(), lse.data_ptr()))
+                g = ctypes.c_void_p()
+                L.check(f.tn_stream_end_capture(stream, ctypes.byref(g)))
+                for _ in range(2):
+                    out.zero_()
+                    tn.synchronize()
+                    L.check(f.tn_graph_launch(stream, g))
+                    L.check(f.tn_stream_synchronize(stream))
+                    assert same((out.bits(), lse.numpy())), (stream is bare, fn)
+                L.check(f.tn_graph_destroy(g))
+        assert tn._hip_counters()["workspace_bytes"] == before
+    finally:
+        L.check(f.tn_stream_destroy(bare))
+        L.check(f.tn_stream_destroy(held))
 
 
 def test_noalloc_refuses_a_call_larger_than_its_array(tn):

@@ -6,8 +6,9 @@
 namespace tn {
 
 bool decode_any_f32_takes(int64_t Hq, int64_t D);
-// The splits it would like; the caller provides the partials (part_o B*Hq*nsplit
-// rows of D floats, part_ml as many pairs) or passes 1.
+// The splits it takes (the result's bits depend on them); the caller provides the
+// partials (part_o B*Hq*nsplit rows of D floats, part_ml as many pairs) if it can:
+// without them one workgroup takes all the splits of its rows.
 int decode_any_f32_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t max_len);
 // Pointers 16-byte aligned; lens, B, Hq, cap and max_len as tn_sdpa_decode checks them.
 tn_status decode_any_f32(hipStream_t st, const float* q, const float* k, const float* v, int64_t B, int64_t Hq,

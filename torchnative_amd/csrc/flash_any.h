@@ -15,9 +15,9 @@ struct AnyArgs {
     int causal;
     const int32_t* lens;  // nullable [B]: keys of sequence b (at most max_len and S)
     int max_len;
-    int nsplit;        // splits of the keys; above 1 the partials below hold
+    int nsplit;        // splits of the keys (the result's bits depend on it); above 1 the partials below hold
     float* part_o;     // BH * L * nsplit * D floats and
-    float2* part_ml;   // BH * L * nsplit pairs
+    float2* part_ml;   // BH * L * nsplit pairs; null: a workgroup takes its row's splits one after another
     int mk;            // mask kind: 0 none, 1 f32, 2 the input format, 3 bool
     int mahead;        // its quads are loaded with their keys (mask_ahead)
     const void* mask;  // and its element strides over (B, Hq, L, S)
@@ -28,7 +28,7 @@ constexpr int FLASH_ANY_MAX_SPLIT = 64;
 
 // Whether the kernel takes this call (head dim, alignment, sizes).
 bool flash_any_takes(const AnyArgs& a);
-// The splits it would like; the caller provides the partials or sets 1.
+// The splits it takes; the caller provides partials for them if it can.
 int flash_any_splits(const AnyArgs& a);
 tn_status flash_any_launch(hipStream_t st, bool f16, const AnyArgs& a);
 

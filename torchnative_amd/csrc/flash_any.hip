@@ -86,7 +86,24 @@ __device__ __attribute__((always_inline)) inline uint32_t finite2(uint32_t w) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), (u16x2){LOW, LOW}));
 }
 
-template <int DT, int NQ, bool MASKED, bool F16>
+// The merge of a row's splits, one after another in split order from
+// m = -inf, l = 0, o = 0: o = o * a + o_s * b, l likewise. k_any_combine and the
+// kernel that takes its splits in turn (SEQ) give the same bits.
+struct SplitMerge {
+    float a, b;
+    __device__ __attribute__((always_inline)) inline SplitMerge(float2 s, float& m, float& l) {
+        const float mn = fmaxf(m, s.x);
+        const float mu = mn == -INFINITY ? 0.0f : mn;
+        a = exp2f(m - mu);
+        b = exp2f(s.x - mu);
+        l = l * a + s.y * b;
+        m = mn;
+    }
+    __device__ __attribute__((always_inline)) inline float operator()(float o, float os) const { return o * a + os * b; }
+};
+
+// SEQ: no partials, one workgroup takes all the splits of its rows.
+template <int DT, int NQ, bool MASKED, bool F16, bool SEQ>
 __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArgs a) {
     using C = AnyCfg<DT, NQ>;
     using E = El<F16>;
@@ -102,8 +119,8 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
     const int lq = lane & 31, hh = lane >> 5;
     // long causal blocks first; the splits of a block side by side
     const int nqb = (a.L + C::BQ - 1) / C::BQ;
-    const int split = (int)blockIdx.x % a.nsplit;
-    const int unit = (int)blockIdx.x / a.nsplit;
+    int split = SEQ ? 0 : (int)blockIdx.x % a.nsplit;
+    const int unit = SEQ ? (int)blockIdx.x : (int)blockIdx.x / a.nsplit;
     const int bh = unit % a.BH, qt = nqb - 1 - unit / a.BH;
     const int h = bh % a.Hq, b = bh / a.Hq;
     const int kvh = h / (a.Hq / a.Hkv);
@@ -112,8 +129,6 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
     const int kvalid = a.lens ? max(0, min(min(a.lens[b], a.max_len), a.S)) : a.S;
     const int kend = a.causal ? min(kvalid, q0 + C::BQ) : kvalid;
     const int nst_row = (kend + C::ROWS - 1) / C::ROWS;
-    const int st_lo = (int)((int64_t)split * nst_row / a.nsplit);
-    const int st_hi = (int)((int64_t)(split + 1) * nst_row / a.nsplit);
 
     const uint16_t* qp = a.q + (int64_t)bh * a.L * D;
     const uint16_t* kp = a.k + ((int64_t)b * a.Hkv + kvh) * a.S * D;
@@ -169,167 +184,195 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
     };
 
     f32x16 o[DT];
+    float m, l;
+    [[maybe_unused]] f32x16 so[SEQ ? DT : 1];  // SEQ: the splits so far
+    [[maybe_unused]] float sm = -INFINITY, sl = 0.0f;
+    if constexpr (SEQ) {
 #pragma unroll
-    for (int i = 0; i < DT; i++)
+        for (int i = 0; i < DT; i++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[i][r] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
-    if (st_lo < st_hi) {
-        issue(st_lo);
-        mload(st_lo);
+            for (int r = 0; r < 16; r++) so[i][r] = 0.0f;
     }
-    for (int st = st_lo; st < st_hi; st++) {
-        wait_vmcnt<0>();  // the only loads in flight are this stage's
-        if constexpr (MASKED) {
+    do {
+        if (SEQ && split > 0) __syncthreads();  // the last split's merge has read the ring
 #pragma unroll
-            for (int rq = 0; rq < 4; rq++) {
-                // the compiler's own wait falls here, where nothing is in flight
-                asm volatile("" : "+v"(mq[rq]));
-                mcur[rq] = mq[rq];
+        for (int i = 0; i < DT; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[i][r] = 0.0f;
+        m = -INFINITY, l = 0.0f;
+        const int st_lo = (int)((int64_t)split * nst_row / a.nsplit);
+        const int st_hi = (int)((int64_t)(split + 1) * nst_row / a.nsplit);
+        if (st_lo < st_hi) {
+            issue(st_lo);
+            mload(st_lo);
+        }
+        for (int st = st_lo; st < st_hi; st++) {
+            wait_vmcnt<0>();  // the only loads in flight are this stage's
+            if constexpr (MASKED) {
+#pragma unroll
+                for (int rq = 0; rq < 4; rq++) {
+                    // the compiler's own wait falls here, where nothing is in flight
+                    asm volatile("" : "+v"(mq[rq]));
+                    mcur[rq] = mq[rq];
+                }
             }
-        }
-        // this wave's reads of the other stage, which the barrier opens to issue()
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (st + 1 < st_hi) {
-            issue(st + 1);  // into the stage read before the barrier
-            mload(st + 1);
-        }
-        const int k0 = st * C::ROWS + kg * 32;
-        if (k0 >= kend || (a.causal && qw0 + 31 < k0)) continue;
-        const uint16_t* tK = reinterpret_cast<const uint16_t*>(ring + (st & 1) * 2 * C::STAGE);
-        const uint16_t* tV = tK + C::STAGE / 2;
-        const int kr = 32 * kg;
+            // this wave's reads of the other stage, which the barrier opens to issue()
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (st + 1 < st_hi) {
+                issue(st + 1);  // into the stage read before the barrier
+                mload(st + 1);
+            }
+            const int k0 = st * C::ROWS + kg * 32;
+            if (k0 >= kend || (a.causal && qw0 + 31 < k0)) continue;
+            const uint16_t* tK = reinterpret_cast<const uint16_t*>(ring + (st & 1) * 2 * C::STAGE);
+            const uint16_t* tV = tK + C::STAGE / 2;
+            const int kr = 32 * kg;
 
-        f32x16 acc;
+            f32x16 acc;
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+            for (int r = 0; r < 16; r++) acc[r] = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 2 * DT; c++) {
-            const int row = kr + lq;
-            const V8 ka = *reinterpret_cast<const V8*>(tK + row * P + swz(row, 2 * c + hh) * 8);
-            acc = E::mfma(ka, qf[c], acc);
-        }
-        // the XDL wait states before VALU reads the products (as k_flash16)
-        asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(acc));
-        float v[16];
+            for (int c = 0; c < 2 * DT; c++) {
+                const int row = kr + lq;
+                const V8 ka = *reinterpret_cast<const V8*>(tK + row * P + swz(row, 2 * c + hh) * 8);
+                acc = E::mfma(ka, qf[c], acc);
+            }
+            // the XDL wait states before VALU reads the products (as k_flash16)
+            asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(acc));
+            float v[16];
 #pragma unroll
-        for (int r = 0; r < 16; r++) v[r] = acc[r] * a.sl2;
-        if constexpr (MASKED) {
-            if (a.mahead) {
+            for (int r = 0; r < 16; r++) v[r] = acc[r] * a.sl2;
+            if constexpr (MASKED) {
+                if (a.mahead) {
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    const f32x4 mv = any_mask_values<F16>(a.mk, mcur[rq], mr.shift);
+                    for (int rq = 0; rq < 4; rq++) {
+                        const f32x4 mv = any_mask_values<F16>(a.mk, mcur[rq], mr.shift);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] + mv[e] * LOG2E;
+                        for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] + mv[e] * LOG2E;
+                    }
+                } else if (qi < a.L) {
+                    const int64_t mrow = (int64_t)b * mask.sb + (int64_t)h * mask.sh + (int64_t)qi * mask.sl;
+#pragma unroll
+                    for (int rq = 0; rq < 4; rq++) {
+                        const f32x4 mv = any_mask_quad<F16>(a.mk, mask, mrow, k0 + 8 * rq + 4 * hh, a.S);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] + mv[e] * LOG2E;
+                    }
                 }
-            } else if (qi < a.L) {
-                const int64_t mrow = (int64_t)b * mask.sb + (int64_t)h * mask.sh + (int64_t)qi * mask.sl;
+            }
+            if (k0 + 32 > kvalid || (a.causal && k0 + 31 > qw0)) {
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    const f32x4 mv = any_mask_quad<F16>(a.mk, mask, mrow, k0 + 8 * rq + 4 * hh, a.S);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[4 * rq + e] = v[4 * rq + e] + mv[e] * LOG2E;
+                for (int r = 0; r < 16; r++) {
+                    const int key = k0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+                    if (key >= kvalid || (a.causal && key > qi)) v[r] = -INFINITY;
                 }
             }
-        }
-        if (k0 + 32 > kvalid || (a.causal && k0 + 31 > qw0)) {
+            float mx = max3f(max3f(max3f(v[0], v[1], v[2]), v[3], v[4]), max3f(v[5], v[6], v[7]),
+                             max3f(max3f(v[8], v[9], v[10]), v[11], v[12]));
+            mx = xor32_max(max3f(mx, max3f(v[13], v[14], v[15]), mx));
+            const bool need = mx > m + RESCALE_SLACK;
+            if (__any(need)) {
+                const float mn = need ? mx : m;
+                // a row with no key seen yet keeps m = mn = -inf: alpha 1, not 2^NaN
+                const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+                l = l * alpha;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int key = k0 + 8 * (r >> 2) + 4 * hh + (r & 3);
-                if (key >= kvalid || (a.causal && key > qi)) v[r] = -INFINITY;
+                for (int i = 0; i < DT; i++) o[i] = o[i] * alpha;
+                m = mn;
             }
-        }
-        float mx = max3f(max3f(max3f(v[0], v[1], v[2]), v[3], v[4]), max3f(v[5], v[6], v[7]),
-                         max3f(max3f(v[8], v[9], v[10]), v[11], v[12]));
-        mx = xor32_max(max3f(mx, max3f(v[13], v[14], v[15]), mx));
-        const bool need = mx > m + RESCALE_SLACK;
-        if (__any(need)) {
-            const float mn = need ? mx : m;
-            // a row with no key seen yet keeps m = mn = -inf: alpha 1, not 2^NaN
-            const float alpha = mn == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
-            l = l * alpha;
+            const float mu = ((m == -INFINITY) ? 0.0f : m) - P_BIAS<F16>;
+            float p[16];
 #pragma unroll
-            for (int i = 0; i < DT; i++) o[i] = o[i] * alpha;
-            m = mn;
-        }
-        const float mu = ((m == -INFINITY) ? 0.0f : m) - P_BIAS<F16>;
-        float p[16];
+            for (int r = 0; r < 16; r++) p[r] = __builtin_amdgcn_exp2f(v[r] - mu);
+            float ps = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; r++) p[r] = __builtin_amdgcn_exp2f(v[r] - mu);
-        float ps = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; r += 4) ps = ps + ((p[r] + p[r + 1]) + (p[r + 2] + p[r + 3]));
-        l = l + ps;
-        V8 ph[2], pl[2];  // p = hi + lo
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            uint32_t hi[4], lo[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float x0 = p[8 * j + 2 * e], x1 = p[8 * j + 2 * e + 1];
-                hi[e] = E::pack_p(hi_of<F16>(x0), hi_of<F16>(x1));
-                lo[e] = E::pack_p(x0 - E::lo(hi[e]), x1 - E::hi(hi[e]));
-            }
-            ph[j] = __builtin_bit_cast(V8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-            pl[j] = __builtin_bit_cast(V8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
-        }
-        const int gi = lane & 15;
-        const int dcol = 16 * ((lane >> 4) & 1) + 4 * (gi & 3);  // the V^T operand's source columns (k_flash16)
-#pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
+            for (int r = 0; r < 16; r += 4) ps = ps + ((p[r] + p[r + 1]) + (p[r + 2] + p[r + 3]));
+            l = l + ps;
+            V8 ph[2], pl[2];  // p = hi + lo
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                const int r0 = kr + 16 * j + 4 * hh + (gi >> 2), r1 = r0 + 8;
-                const int col = 32 * dt + dcol;
-                const uint2 lo = lds_read_tr16(tV + r0 * P + swz(r0, col >> 3) * 8 + (col & 7));
-                const uint2 hi = lds_read_tr16(tV + r1 * P + swz(r1, col >> 3) * 8 + (col & 7));
-                const V8 va = __builtin_bit_cast(V8, make_uint4(lo.x, lo.y, hi.x, hi.y));
-                const V8 vf = __builtin_bit_cast(V8, make_uint4(finite2<F16>(lo.x), finite2<F16>(lo.y),
-                                                                finite2<F16>(hi.x), finite2<F16>(hi.y)));
-                o[dt] = E::mfma(va, ph[j], o[dt]);
-                o[dt] = E::mfma(vf, pl[j], o[dt]);
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float x0 = p[8 * j + 2 * e], x1 = p[8 * j + 2 * e + 1];
+                    hi[e] = E::pack_p(hi_of<F16>(x0), hi_of<F16>(x1));
+                    lo[e] = E::pack_p(x0 - E::lo(hi[e]), x1 - E::hi(hi[e]));
+                }
+                ph[j] = __builtin_bit_cast(V8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                pl[j] = __builtin_bit_cast(V8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+            }
+            const int gi = lane & 15;
+            const int dcol = 16 * ((lane >> 4) & 1) + 4 * (gi & 3);  // the V^T operand's source columns (k_flash16)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const int r0 = kr + 16 * j + 4 * hh + (gi >> 2), r1 = r0 + 8;
+                    const int col = 32 * dt + dcol;
+                    const uint2 lo = lds_read_tr16(tV + r0 * P + swz(r0, col >> 3) * 8 + (col & 7));
+                    const uint2 hi = lds_read_tr16(tV + r1 * P + swz(r1, col >> 3) * 8 + (col & 7));
+                    const V8 va = __builtin_bit_cast(V8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                    const V8 vf = __builtin_bit_cast(V8, make_uint4(finite2<F16>(lo.x), finite2<F16>(lo.y),
+                                                                    finite2<F16>(hi.x), finite2<F16>(hi.y)));
+                    o[dt] = E::mfma(va, ph[j], o[dt]);
+                    o[dt] = E::mfma(vf, pl[j], o[dt]);
+                }
             }
         }
-    }
 #pragma unroll
-    for (int i = 0; i < DT; i++) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(o[i]));
+        for (int i = 0; i < DT; i++) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(o[i]));
 
-    l = xor32_sum(l);
-    // tree merge of the key groups through LDS, over the ring (every load has
-    // landed and been read once the first barrier has passed)
-    constexpr int WSLOT = DT * 16 * 64;  // floats per wave
-    static_assert((KG / 2) * NQ * WSLOT * 4 <= 4 * C::STAGE, "merge slots must fit in the ring");
+        l = xor32_sum(l);
+        // tree merge of the key groups through LDS, over the ring (every load has
+        // landed and been read once the first barrier has passed)
+        constexpr int WSLOT = DT * 16 * 64;  // floats per wave
+        static_assert((KG / 2) * NQ * WSLOT * 4 <= 4 * C::STAGE, "merge slots must fit in the ring");
 #pragma unroll
-    for (int half = KG / 2; half >= 1; half /= 2) {
-        __syncthreads();
-        if (kg >= half && kg < 2 * half) {
-            float* xo = reinterpret_cast<float*>(ring) + ((kg - half) * NQ + qw) * WSLOT;
+        for (int half = KG / 2; half >= 1; half /= 2) {
+            __syncthreads();
+            if (kg >= half && kg < 2 * half) {
+                float* xo = reinterpret_cast<float*>(ring) + ((kg - half) * NQ + qw) * WSLOT;
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++)
+                for (int dt = 0; dt < DT; dt++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) xo[(dt * 16 + r) * 64 + lane] = o[dt][r];
-            s_ml[kg - half][qw][lane] = make_float2(m, l);
+                    for (int r = 0; r < 16; r++) xo[(dt * 16 + r) * 64 + lane] = o[dt][r];
+                s_ml[kg - half][qw][lane] = make_float2(m, l);
+            }
+            __syncthreads();
+            if (kg < half) {
+                const float* xo = reinterpret_cast<const float*>(ring) + (kg * NQ + qw) * WSLOT;
+                const float2 ml1 = s_ml[kg][qw][lane];
+                const float mm = fmaxf(m, ml1.x);
+                const float mu = (mm == -INFINITY) ? 0.0f : mm;
+                const float a0 = __builtin_amdgcn_exp2f(m - mu), a1 = __builtin_amdgcn_exp2f(ml1.x - mu);
+                l = l * a0 + ml1.y * a1;
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) o[dt][r] = o[dt][r] * a0 + xo[(dt * 16 + r) * 64 + lane] * a1;
+                m = mm;
+            }
         }
-        __syncthreads();
-        if (kg < half) {
-            const float* xo = reinterpret_cast<const float*>(ring) + (kg * NQ + qw) * WSLOT;
-            const float2 ml1 = s_ml[kg][qw][lane];
-            const float mm = fmaxf(m, ml1.x);
-            const float mu = (mm == -INFINITY) ? 0.0f : mm;
-            const float a0 = __builtin_amdgcn_exp2f(m - mu), a1 = __builtin_amdgcn_exp2f(ml1.x - mu);
-            l = l * a0 + ml1.y * a1;
+        if constexpr (SEQ) {
+            if (kg == 0) {
+                const SplitMerge mg(make_float2(m, l), sm, sl);
 #pragma unroll
-            for (int dt = 0; dt < DT; dt++)
+                for (int i = 0; i < DT; i++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[dt][r] = o[dt][r] * a0 + xo[(dt * 16 + r) * 64 + lane] * a1;
-            m = mm;
+                    for (int r = 0; r < 16; r++) so[i][r] = mg(so[i][r], o[i][r]);
+            }
         }
+    } while (SEQ && ++split < a.nsplit);
+    if constexpr (SEQ) {
+#pragma unroll
+        for (int i = 0; i < DT; i++) o[i] = so[i];
+        m = sm, l = sl;
     }
     if (kg != 0 || qi >= a.L) return;
     const int64_t row = (int64_t)bh * a.L + qi;
-    if (a.nsplit > 1) {
+    if (!SEQ && a.nsplit > 1) {
         float* po = a.part_o + (row * a.nsplit + split) * D;
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
@@ -369,32 +412,25 @@ __global__ __launch_bounds__(256) void k_any_combine(const AnyArgs a, int64_t ro
     const int64_t row = t / q4;
     const int c = (int)(t - row * q4) * 4;
     if (row >= rows) return;
-    float mm = -INFINITY;
-    for (int s = 0; s < a.nsplit; s++) mm = fmaxf(mm, a.part_ml[row * a.nsplit + s].x);
-    const float mu = mm == -INFINITY ? 0.0f : mm;
-    float tl = 0.0f;
+    float mm = -INFINITY, tl = 0.0f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
     for (int s = 0; s < a.nsplit; s++) {
-        const float2 ml = a.part_ml[row * a.nsplit + s];
         const float4 v = *reinterpret_cast<const float4*>(a.part_o + (row * a.nsplit + s) * a.D + c);
-        const float f = exp2f(ml.x - mu);
-        tl = tl + ml.y * f;
-        acc.x = acc.x + v.x * f;
-        acc.y = acc.y + v.y * f;
-        acc.z = acc.z + v.z * f;
-        acc.w = acc.w + v.w * f;
+        const SplitMerge mg(a.part_ml[row * a.nsplit + s], mm, tl);
+        acc = make_float4(mg(acc.x, v.x), mg(acc.y, v.y), mg(acc.z, v.z), mg(acc.w, v.w));
     }
     const float inv = 1.0f / tl;
     *reinterpret_cast<uint2*>(a.out + row * a.D + c) =
         make_uint2(El<F16>::pack_out(acc.x * inv, acc.y * inv), El<F16>::pack_out(acc.z * inv, acc.w * inv));
     if (a.lse && c == 0)
-        a.lse[row] = mm == -INFINITY ? (a.lens ? -INFINITY : NAN) : mu * LN2 + logf(tl * P_UNIT<F16>);
+        a.lse[row] = mm == -INFINITY ? (a.lens ? -INFINITY : NAN) : mm * LN2 + logf(tl * P_UNIT<F16>);
 }
 
-template <int DT, int NQ>
+template <int DT, int NQ, bool SEQ>
 void launch_nq(hipStream_t st, const AnyArgs& a, bool f16, unsigned grid) {
     using C = AnyCfg<DT, NQ>;
-#define TN_FA(M, H) hipLaunchKernelGGL((k_flash_any<DT, NQ, M, H>), dim3(grid), dim3(C::NT), 0, st, a)
+#define TN_FA(M, H) hipLaunchKernelGGL((k_flash_any<DT, NQ, M, H, SEQ>), dim3(grid), dim3(C::NT), 0, st, a)
     if (a.mk) {
         if (f16) TN_FA(true, true);
         else TN_FA(true, false);
@@ -407,9 +443,14 @@ void launch_nq(hipStream_t st, const AnyArgs& a, bool f16, unsigned grid) {
 
 template <int DT>
 void launch_dt(hipStream_t st, const AnyArgs& a, bool f16, int nq) {
-    const unsigned grid = (unsigned)((int64_t)a.BH * cdiv(a.L, 32 * nq) * a.nsplit);
-    if (nq == 1) launch_nq<DT, 1>(st, a, f16, grid);
-    else launch_nq<DT, 2>(st, a, f16, grid);
+    const unsigned units = (unsigned)((int64_t)a.BH * cdiv(a.L, 32 * nq));
+    if (a.nsplit > 1 && !a.part_o) {
+        if (nq == 1) launch_nq<DT, 1, true>(st, a, f16, units);
+        else launch_nq<DT, 2, true>(st, a, f16, units);
+    } else {
+        if (nq == 1) launch_nq<DT, 1, false>(st, a, f16, units * a.nsplit);
+        else launch_nq<DT, 2, false>(st, a, f16, units * a.nsplit);
+    }
 }
 
 }  // namespace
@@ -439,7 +480,7 @@ tn_status flash_any_launch(hipStream_t st, bool f16, const AnyArgs& a) {
     else if (dt == 4) launch_dt<4>(st, a, f16, nq);
     else launch_dt<8>(st, a, f16, nq);
     TN_LAUNCHED();
-    if (a.nsplit > 1) {
+    if (a.nsplit > 1 && a.part_o) {
         const int64_t rows = (int64_t)a.BH * a.L;
         const dim3 grid((unsigned)cdiv(rows * (a.D / 4), 256));
         if (f16) hipLaunchKernelGGL(k_any_combine<true>, grid, dim3(256), 0, st, a, rows);

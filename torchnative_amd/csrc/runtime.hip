@@ -126,6 +126,19 @@ tn_status workspace_or_none(hipStream_t stream, size_t bytes, void** out) {
     return workspace(stream, bytes, out);
 }
 
+tn_status workspace_if_held(hipStream_t stream, size_t bytes, void** out) {
+    *out = nullptr;
+    int dev = 0;
+    TN_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(g_ws_mu);
+    const auto it = g_ws.find({dev, stream});
+    if (it == g_ws.end() || it->second.bytes < bytes) return TN_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    TN_HIP(hipStreamIsCapturing(stream, &cs));
+    if (cs == hipStreamCaptureStatusNone) *out = it->second.ptr;
+    return TN_OK;
+}
+
 tn_status tickets(hipStream_t stream, size_t n, uint32_t** out) {
     int dev = 0;
     TN_HIP(hipGetDevice(&dev));

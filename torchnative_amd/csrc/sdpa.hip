@@ -2038,23 +2038,24 @@ tn_status decode_check(int dtype, int64_t B, int64_t Hq, int64_t Hkv, int64_t ca
 }
 
 // Decode attention at the head dims other than 64 and 128: flash_any for 16-bit
-// caches and decode_any_f32 for f32 ones (the partials, if given, hold max_split
-// splits of B * Hq rows), otherwise the plain kernel, one query row per
-// (sequence, head) over the cache's cap rows.
+// caches and decode_any_f32 for f32 ones (at most max_split splits; the partials,
+// if given, hold that many of B * Hq rows, and without them the bits are the
+// same), otherwise the plain kernel, one query row per (sequence, head) over the
+// cache's cap rows.
 static tn_status decode_any(hipStream_t st, int dtype, const void* q, const void* k_cache, const void* v_cache, int64_t B,
                             int64_t Hq, int64_t Hkv, int64_t cap, int64_t D, const int32_t* lens, int64_t max_len,
                             double sc, void* out, float* lse, float* part_o, float2* part_ml, int max_split) {
     if (dtype != TN_F32) {
         AnyArgs a = decode_any_args(q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse);
         if (flash_any_takes(a)) {
-            a.nsplit = part_o ? std::min(max_split, flash_any_splits(a)) : 1;
+            a.nsplit = std::min(max_split, flash_any_splits(a));
             a.part_o = part_o;
             a.part_ml = part_ml;
             return flash_any_launch(st, dtype == TN_F16, a);
         }
     }
     if (dtype == TN_F32 && decode_any_f32_takes(Hq, D)) {
-        const int ns = part_o ? std::min(max_split, decode_any_f32_splits(B, Hq, Hkv, D, max_len)) : 1;
+        const int ns = std::min(max_split, decode_any_f32_splits(B, Hq, Hkv, D, max_len));
         return decode_any_f32(st, static_cast<const float*>(q), static_cast<const float*>(k_cache),
                               static_cast<const float*>(v_cache), B, Hq, Hkv, cap, D, lens, max_len, sc,
                               static_cast<float*>(out), lse, part_o, part_ml, ns);
@@ -2533,12 +2534,13 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
                 const int ns = flash_any_splits(a);
                 if (ns > 1) {
                     // split keys when the rows alone leave the device idle; under a
-                    // capture that could not grow the workspace, unsplit
+                    // capture that could not grow the workspace a workgroup takes
+                    // its rows' splits in turn, the same bits
                     const size_t po = (size_t)rows * ns * D * sizeof(float), pm = (size_t)rows * ns * sizeof(float2);
                     void* ws = nullptr;
                     TN_TRY(workspace_or_none(st, po + pm, &ws));
+                    a.nsplit = ns;
                     if (ws) {
-                        a.nsplit = ns;
                         a.part_o = static_cast<float*>(ws);
                         a.part_ml = reinterpret_cast<float2*>(static_cast<char*>(ws) + po);
                     }
@@ -2706,13 +2708,13 @@ tn_status decode_entry(void* stream, int dtype, const void* q, const void* k_cac
             ns = decode_any_f32_splits(B, Hq, Hkv, D, max_len);
         }
         if (ns > 1) {
-            // as many splits as the no-alloc entry's array holds, in either
-            // entry (they give the same bits); none where a capture could not
-            // grow the stream's workspace
-            const size_t one = (size_t)B * Hq * (D * sizeof(float) + sizeof(float2));
-            ns = (int)std::min<size_t>(ns, DECODE_SCRATCH_BYTES / one);
+            // either entry gives these splits' bits whatever the stream holds: with no
+            // partials (a capture that could not grow the workspace; the no-alloc
+            // entry, which takes no more than the stream has) one workgroup takes its
+            // rows' splits in turn. Neither uses the GPU's shared array.
             po = (size_t)B * Hq * ns * D * sizeof(float);
-            if (ns > 1) TN_TRY((get == workspace ? workspace_or_none : get)(st, one * ns, &ws));
+            const size_t bytes = po + (size_t)B * Hq * ns * sizeof(float2);
+            TN_TRY((get == workspace ? workspace_or_none : workspace_if_held)(st, bytes, &ws));
         }
         return decode_any(st, dtype, q, k_cache, v_cache, B, Hq, Hkv, cap, D, lens, max_len, sc, out, lse,
                           static_cast<float*>(ws), ws ? reinterpret_cast<float2*>(static_cast<char*>(ws) + po) : nullptr,

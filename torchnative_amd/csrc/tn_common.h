@@ -36,6 +36,9 @@ tn_status workspace(hipStream_t stream, size_t bytes, void** out);
 // The same for a call that can do without: null, and no refusal, where the
 // stream is under graph capture and its workspace would have to grow.
 tn_status workspace_or_none(hipStream_t stream, size_t bytes, void** out);
+// For a call that may not allocate: null unless the stream holds that much and is
+// not under graph capture (a graph could outlive the buffer).
+tn_status workspace_if_held(hipStream_t stream, size_t bytes, void** out);
 // Per-(device, stream) array of n uint32 counters, zero when first handed out
 // (cleared on the stream at allocation). A kernel that takes tickets from it
 // must leave every counter at zero again when it ends.
