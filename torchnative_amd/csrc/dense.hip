@@ -140,8 +140,7 @@ constexpr int DL_XCD = 8;
 
 // tiles numbered down the rows first, consecutive numbers on one XCD (its
 // workgroups share the columns of w in its L2)
-__device__ inline int dense_wg() {
-    const int nwg = (int)gridDim.x, id = (int)blockIdx.x;
+__device__ inline int dense_wg(int id, int nwg) {
     return nwg % DL_XCD == 0 ? (id % DL_XCD) * (nwg / DL_XCD) + id / DL_XCD : id;
 }
 
@@ -159,10 +158,11 @@ template <int WT>
 __global__ void __launch_bounds__(DL_THREADS) k_dense_any(const float* __restrict__ x, int M, int K,
                                                           const void* __restrict__ w, int N,
                                                           const float* __restrict__ bias, float* __restrict__ y,
-                                                          int mtiles, int ntiles) {
+                                                          int mtiles, int ntiles, int nwg) {
     constexpr int RING = 8;
+    if (wg_number() >= nwg) return;
     const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
-    const int64_t tile = (int64_t)dense_wg() * DL_WAVES + (threadIdx.x >> 6);
+    const int64_t tile = (int64_t)dense_wg(wg_number(), nwg) * DL_WAVES + (threadIdx.x >> 6);
     if (tile >= (int64_t)mtiles * ntiles) return;
     const int m0 = (int)(tile % mtiles) * 16, n0 = (int)(tile / mtiles) * 16;
     const float* xr = x + (int64_t)min(m0 + i16, M - 1) * K;
@@ -231,7 +231,8 @@ template <int WT, int WM, int WN, int RT, int CT, int KS, int NS>
 __global__ void __launch_bounds__(DL_THREADS) k_dense_lds(const float* __restrict__ x, int M, int K,
                                                           const void* __restrict__ w, int N,
                                                           const float* __restrict__ bias, float* __restrict__ y,
-                                                          int mtiles) {
+                                                          int mtiles, int nwg) {
+    if (wg_number() >= nwg) return;
     static_assert(WM * WN == DL_WAVES, "waves");
     static_assert(NS >= 3, "ring");
     constexpr int WS = WT == TN_F32 ? 4 : 2;             // bytes of a stored weight
@@ -245,7 +246,7 @@ __global__ void __launch_bounds__(DL_THREADS) k_dense_lds(const float* __restric
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, g = lane >> 4;
-    const int wg = dense_wg();
+    const int wg = dense_wg(wg_number(), nwg);
     const int m0 = wg % mtiles * BM, n0 = wg / mtiles * BN;
     const int wm0 = wave / WN * 16 * RT, wn0 = wave % WN * 16 * CT;  // the wave's first row and column in the tile
 
@@ -383,15 +384,17 @@ void launch_dense(hipStream_t st, const float* x, int64_t M, int64_t K, const vo
     const bool aligned = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0 &&
                          K * WS % 16 == 0 && K % 4 == 0 && 64 * K * 4 <= INT32_MAX;
     if (!aligned || K < 16) {
-        const int64_t mt = cdiv(M, 16), nt = cdiv(N, 16);
-        hipLaunchKernelGGL(k_dense_any<WT>, dim3((unsigned)cdiv(mt * nt, DL_WAVES)), dim3(DL_THREADS), 0, st, x, (int)M,
-                           (int)K, w, (int)N, bias, y, (int)mt, (int)nt);
+        const int64_t mt = cdiv(M, 16), nt = cdiv(N, 16), wgs = cdiv(mt * nt, DL_WAVES);
+        hipLaunchKernelGGL(k_dense_any<WT>, wg_grid(wgs), dim3(DL_THREADS), 0, st, x, (int)M, (int)K, w, (int)N, bias, y,
+                           (int)mt, (int)nt, (int)wgs);
         return;
     }
 #define TN_DL(WM, WN, RT, CT, KS, NS)                                                                                \
-    hipLaunchKernelGGL((k_dense_lds<WT, WM, WN, RT, CT, KS, NS>),                                                    \
-                       dim3((unsigned)(cdiv(M, 16 * RT * WM) * cdiv(N, 16 * CT * WN))), dim3(DL_THREADS), 0, st, x, \
-                       (int)M, (int)K, w, (int)N, bias, y, (int)cdiv(M, 16 * RT * WM))
+    do {                                                                                                             \
+        const int64_t mt = cdiv(M, 16 * RT * WM), wgs = mt * cdiv(N, 16 * CT * WN);                                 \
+        hipLaunchKernelGGL((k_dense_lds<WT, WM, WN, RT, CT, KS, NS>), wg_grid(wgs), dim3(DL_THREADS), 0, st, x,     \
+                           (int)M, (int)K, w, (int)N, bias, y, (int)mt, (int)wgs);                                  \
+    } while (0)
     // one row tile: the four waves side by side over 64 columns (wider than
     // 16 rows would be padding); 64 x 64 once that gives every CU two
     // workgroups (half the LDS reads per product: [1024, 256] x [3200, 256] 25.2

@@ -18,6 +18,7 @@ struct AnyArgs {
     int nsplit;        // splits of the keys (the result's bits depend on it); above 1 the partials below hold
     float* part_o;     // BH * L * nsplit * D floats and
     float2* part_ml;   // BH * L * nsplit pairs; null: a workgroup takes its row's splits one after another
+    int nwg;           // workgroups (set by the launch)
     int mk;            // mask kind: 0 none, 1 f32, 2 the input format, 3 bool
     int mahead;        // its quads are loaded with their keys (mask_ahead)
     const void* mask;  // and its element strides over (B, Hq, L, S)

@@ -119,8 +119,10 @@ __global__ __launch_bounds__((AnyCfg<DT, NQ>::NT)) void k_flash_any(const AnyArg
     const int lq = lane & 31, hh = lane >> 5;
     // long causal blocks first; the splits of a block side by side
     const int nqb = (a.L + C::BQ - 1) / C::BQ;
-    int split = SEQ ? 0 : (int)blockIdx.x % a.nsplit;
-    const int unit = SEQ ? (int)blockIdx.x : (int)blockIdx.x / a.nsplit;
+    const int wg = wg_number();
+    if (wg >= a.nwg) return;
+    int split = SEQ ? 0 : wg % a.nsplit;
+    const int unit = SEQ ? wg : wg / a.nsplit;
     const int bh = unit % a.BH, qt = nqb - 1 - unit / a.BH;
     const int h = bh % a.Hq, b = bh / a.Hq;
     const int kvh = h / (a.Hq / a.Hkv);
@@ -428,9 +430,11 @@ __global__ __launch_bounds__(256) void k_any_combine(const AnyArgs a, int64_t ro
 }
 
 template <int DT, int NQ, bool SEQ>
-void launch_nq(hipStream_t st, const AnyArgs& a, bool f16, unsigned grid) {
+void launch_nq(hipStream_t st, AnyArgs a, bool f16, int64_t wgs) {
     using C = AnyCfg<DT, NQ>;
-#define TN_FA(M, H) hipLaunchKernelGGL((k_flash_any<DT, NQ, M, H, SEQ>), dim3(grid), dim3(C::NT), 0, st, a)
+    const dim3 grid = wg_grid(wgs);
+    a.nwg = (int)wgs;
+#define TN_FA(M, H) hipLaunchKernelGGL((k_flash_any<DT, NQ, M, H, SEQ>), grid, dim3(C::NT), 0, st, a)
     if (a.mk) {
         if (f16) TN_FA(true, true);
         else TN_FA(true, false);
@@ -443,7 +447,7 @@ void launch_nq(hipStream_t st, const AnyArgs& a, bool f16, unsigned grid) {
 
 template <int DT>
 void launch_dt(hipStream_t st, const AnyArgs& a, bool f16, int nq) {
-    const unsigned units = (unsigned)((int64_t)a.BH * cdiv(a.L, 32 * nq));
+    const int64_t units = (int64_t)a.BH * cdiv(a.L, 32 * nq);
     if (a.nsplit > 1 && !a.part_o) {
         if (nq == 1) launch_nq<DT, 1, true>(st, a, f16, units);
         else launch_nq<DT, 2, true>(st, a, f16, units);

@@ -97,7 +97,7 @@ struct QGeo {
 
 template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS, bool DMA>
 __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf, const float* __restrict__ dxf, int M,
-                                                 int mtiles, int nb, const uint8_t* __restrict__ qs,
+                                                 int mtiles, int nwg, int nb, const uint8_t* __restrict__ qs,
                                                  const uint16_t* __restrict__ dw, int N, const float* __restrict__ bias,
                                                  void* y, int y_bf16, const float* resid) {
     using G = QGeo<FMT, RT, CT, WM, WN, KB, NS>;
@@ -111,7 +111,8 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
     const int i16 = lane & 15, g = lane >> 4;
     // tiles numbered down the rows first, consecutive numbers on one XCD
     const int mwg = (mtiles + G::RTT - 1) / G::RTT;
-    const int nwg = (int)gridDim.x, id = (int)blockIdx.x;
+    const int id = wg_number();
+    if (id >= nwg) return;
     const int wg = nwg % QG_XCD == 0 ? (id % QG_XCD) * (nwg / QG_XCD) + id / QG_XCD : id;
     const int t0 = wg % mwg * G::RTT, n0 = wg / mwg * BN;  // first row tile, first column
     const int wt = wave / WN * RT, wn = wave % WN * 16 * CT;
@@ -348,8 +349,8 @@ __global__ __launch_bounds__(QG_TH) void k_qgemm(const uint8_t* __restrict__ xf,
 template <int FMT, int RT, int CT, int WM, int WN, int KB, int NS, bool DMA = true>
 void launch(hipStream_t st, const QGemmArgs& a, const uint8_t* xf, const float* dxf, int mt, int nb) {
     using G = QGeo<FMT, RT, CT, WM, WN, KB, NS>;
-    const dim3 grid((unsigned)(cdiv(mt, G::RTT) * cdiv(a.n, G::BN)));
-    hipLaunchKernelGGL((k_qgemm<FMT, RT, CT, WM, WN, KB, NS, DMA>), grid, dim3(QG_TH), 0, st, xf, dxf, (int)a.m, mt, nb,
+    const int64_t wgs = cdiv(mt, G::RTT) * cdiv(a.n, G::BN);
+    hipLaunchKernelGGL((k_qgemm<FMT, RT, CT, WM, WN, KB, NS, DMA>), wg_grid(wgs), dim3(QG_TH), 0, st, xf, dxf, (int)a.m, mt, (int)wgs, nb,
                        a.qs, a.d, (int)a.n, a.bias, a.y, a.y_bf16, a.resid);
 }
 

@@ -88,6 +88,16 @@ tn_status flash64_launch(hipStream_t st, bool f16, int mk, const void* mask, int
         if (e_ != hipSuccess) return ::tn::hip_fail(e_, "launch"); \
     } while (0)
 
+// Workgroups numbered in one sequence (wg_number). A dimension of a grid holds
+// under 2^32 threads, and a launch past that runs without an error but not whole:
+// many workgroups go on in y, whose last row may number past n. The kernel is
+// given n and leaves there.
+constexpr int WG_ROW = 1 << 22;
+inline dim3 wg_grid(int64_t n) {
+    return n <= WG_ROW ? dim3((unsigned)n) : dim3(WG_ROW, (unsigned)((n + WG_ROW - 1) / WG_ROW));
+}
+__device__ inline int wg_number() { return (int)(blockIdx.y * WG_ROW + blockIdx.x); }
+
 // ---- raw buffer access ------------------------------------------------------
 
 // Raw buffer descriptor over `bytes` bytes at `base`: offsets at or past the
