@@ -262,3 +262,32 @@ def test_linear_takes_rows_at_any_element(tn, off):
                                               None, y.data_ptr()))
         want = O.dense_linear(x[off:off + m * k].reshape(m, k), wide, None)
         assert y.numpy().tobytes() == want.tobytes(), fmt
+
+
+@pytest.mark.parametrize("fmt", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("m,k,n,off", [
+    # either side of the lines between the two kernels for rows that are no multiple of 16 bytes (64 x 64 blocks: 128,
+    # 256, 640, 1024), block remainders, rows shorter than a stage, and rows of whole stages at an unaligned address
+    (512, 33, 1024, 0), (513, 17, 1000, 0), (513, 40, 1000, 1), (520, 71, 1000, 0), (1025, 9, 1020, 0),
+    (1030, 95, 1025, 0), (1030, 97, 1025, 0), (2000, 13, 1400, 0), (2000, 401, 1290, 0), (2100, 7, 2050, 0),
+    (2100, 45, 2050, 0), (2070, 64, 2001, 1),
+    # short rows of whole 16 bytes, which otherwise go through LDS
+    (1030, 40, 1025, 0), (1030, 48, 1025, 0), (1600, 24, 1700, 0), (2100, 40, 2050, 0)])
+def test_many_short_or_unaligned_rows_bit_for_bit(tn, fmt, m, k, n, off):
+    from torchnative_amd import _lib as L
+
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal(m * k + off).astype(np.float32)
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    w[n // 2] = -0.0
+    xd = _dev(tn, x)
+    q = tn._quantize(_dev(tn, w), fmt)
+    b = rng.standard_normal(n).astype(np.float32) if m % 2 else None
+    bd = _dev(tn, b) if m % 2 else None
+    y = tn.empty((m, n), "float32", "hip")
+    code = {"f32": L.TN_F32, "f16": L.TN_F16, "bf16": L.TN_BF16}[fmt]
+    L.check(L.lib().tn_dense_linear(None, xd.data_ptr() + 4 * off, m, k, q._qs.data_ptr(), code, n,
+                                    bd.data_ptr() if m % 2 else None, y.data_ptr()))
+    rows = np.unique(np.concatenate([[0, 1, m // 2, m - 2, m - 1], rng.integers(0, m, 24)]))
+    want = O.dense_linear(x[off:].reshape(m, k)[rows], tn._dequantize(q).numpy().reshape(n, k), b)
+    assert y.numpy()[rows].tobytes() == want.tobytes()

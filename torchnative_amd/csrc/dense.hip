@@ -6,8 +6,8 @@
 // a weight is the exactness control: QMatMul::from_arc widens it to f32 up
 // front and takes a plain matmul (candle quantized/mod.rs:836-852), so the
 // call must give exactly the bits of the dense linear on the widened weight
-// (quant.rs:273-279). Here both go through one kernel, k_dense_linear, whose
-// every output is one fixed chain: acc = 0, then acc = fma(x[k], w[k], acc)
+// (quant.rs:273-279). Here both go through the same kernels (k_dense_lds,
+// k_dense_any, k_dense_valu), whose every output is one fixed chain: acc = 0, then acc = fma(x[k], w[k], acc)
 // for k = 0, 1, ..., K-1, then acc + bias (the addmm that nn.Linear's bias
 // branch emits, aten.rs:9686-9700, adds the bias once after the product).
 // The chain does not depend on the tiling, the launch or the row count, so
@@ -377,13 +377,115 @@ __global__ void __launch_bounds__(DL_THREADS) k_dense_lds(const float* __restric
     dense_store<RT, CT>(acc, M, m0 + wm0, N, n0 + wn0, lane, bias, y);
 }
 
+constexpr int DV_T = 64;   // rows of x and output features per workgroup
+constexpr int DV_TK = 16;  // k per LDS stage
+constexpr int DV_LD = 68;  // LDS row stride in floats (float4-aligned, staggers the banks)
+
+// The same chain on the VALU, 64 x 64 outputs a workgroup, for many short rows,
+// above all ones that k_dense_lds cannot read (dense_valu). 256 threads; thread (tx, ty) = (t %
+// 16, t / 16) owns rows ty*4..ty*4+3 and features tx*4..tx*4+3. Stage s holds
+// x[:, 16s..16s+15] and w[:, 16s..16s+15] k-major in LDS; only k < K is ever
+// accumulated. An operand element is read once a workgroup where k_dense_any
+// reads it once a 16 x 16 tile.
+template <int WT>
+__global__ void __launch_bounds__(DL_THREADS) k_dense_valu(const float* __restrict__ x, int M, int K,
+                                                           const void* __restrict__ w, int N,
+                                                           const float* __restrict__ bias, float* __restrict__ y) {
+    __shared__ __align__(16) float xs[DV_TK][DV_LD];
+    __shared__ __align__(16) float ws[DV_TK][DV_LD];
+    const int t = threadIdx.x;
+    const int tx = t % 16, ty = t / 16;
+    const int n0 = blockIdx.x * DV_T, m0 = blockIdx.y * DV_T;
+    const int lk = t % DV_TK, lr = t / DV_TK;  // loader: k column, first row (rows lr + 16i)
+    float acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = 0.0f;
+    for (int k0 = 0; k0 < K; k0 += DV_TK) {
+        const int kk = k0 + lk;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = lr + 16 * i;
+            const int m = m0 + r, n = n0 + r;
+            xs[lk][r] = (m < M && kk < K) ? x[(int64_t)m * K + kk] : 0.0f;
+            ws[lk][r] = (n < N && kk < K) ? widen_w<WT>(w, (int64_t)n * K + kk) : 0.0f;
+        }
+        __syncthreads();
+        const int kend = min(DV_TK, K - k0);  // the same for every thread
+        for (int k = 0; k < kend; k++) {
+            const float4 a = *reinterpret_cast<const float4*>(&xs[k][ty * 4]);
+            const float4 b = *reinterpret_cast<const float4*>(&ws[k][tx * 4]);
+            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_fmaf(av[i], bv[j], acc[i][j]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int m = m0 + ty * 4 + i;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int n = n0 + tx * 4 + j;
+            if (n < N) y[(int64_t)m * N + n] = bias ? acc[i][j] + bias[n] : acc[i][j];
+        }
+    }
+}
+
+// Whether k_dense_valu takes rows that k_dense_lds cannot read. It keeps a few
+// waves on a CU waiting for one LDS buffer, whatever the shape: about 0.145 us a k
+// up to 1024 workgroups, and 9 us to store 64 MB. k_dense_any has 16 times as many
+// tiles and pays for each element it loads, twice that where the rows start at
+// nearly the same place of the memory's lines (K one off a multiple of 32), and a
+// quarter more where a 16-bit weight's odd rows start between dwords. Measured,
+// us, valu / any, f32 weights unless stated, by workgroups here:
+//    108 [333, K] x [1111, K]:  K 17 5.9/4.4  33 8.0/6.1  129 22.5/9.6
+//    256 [1024, K] x [1024, K]: K 13 5.3/4.3  17 6.2/6.5  33 8.2/9.9  45 9.3/7.9  75 14.4/8.4
+//                               129 22.7/17.0   f16: 33 8.5/10.0  63 11.7/13.3  129 23.0/22.1
+//    480 [900, K] x [2000, K]:  K 21 7.8/10.8  45 10.5/12.1  99 18.5/11.8  129 22.8/27.8  299 46.9/29.3
+//                               f16: 99 18.8/14.2  257 41.6/53.3  515 80/51
+//    832 [1000, K] x [3300, K]: K 13 10.5/9.9  33 15.0/30.0  99 24.9/19.5  299 58/53  515 102/78
+//                               f16: 299 62/65  450 93/66  515 102/92
+//   1024 [1024, K] x [4096, K]: K 8 10.4/14.2  33 14.3/35.7  299 52/57  515 93/81   f16: 515 101/110
+//   1760 [1000, K] x [7000, K]: K 13 15.7/17.6  129 40/98  299 77/107  1030 243/317
+// Under eight steps the store is all there is (K 7, 1024 workgroups: 10.2/9.3).
+// `lds`: rows that k_dense_lds reads. It loses where a workgroup has little more
+// than one stage, most of it the last K % 16 steps (us, valu / lds, f32; f16 alike
+// but for the last two):
+//    480 [900, K] x [2000, K]:  K 16 6.8/8.4  24 8.0/11.5  40 10.0/11.8  48 10.7/9.3
+//    640 [1000, K] x [2500, K]: K 16 8.8/9.1  24 10.2/12.1  32 10.8/9.8   f16: 16 8.9/6.6
+//   1760 [1000, K] x [7000, K]: K 24 17.9/23.8  40 20.6/25.5  48 22.6/20.9   f16: 40 22.0/21.0
+inline bool dense_valu(int64_t M, int64_t N, int64_t K, bool lds, bool f32) {
+    const int64_t wgs = cdiv(M, DV_T) * cdiv(N, DV_T);
+    if (wgs <= 128 || K < 8) return false;
+    if (lds) {
+        if (wgs <= 256 || K >= 64) return false;
+        if (wgs < 512) return K < 48;
+        return wgs > 512 && (K < 32 ? f32 || K >= 24 : f32 && K % 16 && wgs > 1024);
+    }
+    const bool same = (K + 1) % 32 <= 2;
+    if (wgs <= 256) return K >= 16 && K < (same ? 72 : 40);
+    if (wgs <= 640) return K < 96 || same;
+    return wgs > 1024 || K < 400 || same || (!f32 && K % 2);
+}
+
 template <int WT>
 void launch_dense(hipStream_t st, const float* x, int64_t M, int64_t K, const void* w, int64_t N, const float* bias,
                   float* y) {
     constexpr int WS = WT == TN_F32 ? 4 : 2;
     const bool aligned = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0 &&
                          K * WS % 16 == 0 && K % 4 == 0 && 64 * K * 4 <= INT32_MAX;
-    if (!aligned || K < 16) {
+    const bool lds = aligned && K >= 16;
+    if (dense_valu(M, N, K, lds, WS == 4)) {
+        hipLaunchKernelGGL(k_dense_valu<WT>, dim3((unsigned)cdiv(N, DV_T), (unsigned)cdiv(M, DV_T)), dim3(DL_THREADS), 0,
+                           st, x, (int)M, (int)K, w, (int)N, bias, y);
+        return;
+    }
+    if (!lds) {
         const int64_t mt = cdiv(M, 16), nt = cdiv(N, 16), wgs = cdiv(mt * nt, DL_WAVES);
         hipLaunchKernelGGL(k_dense_any<WT>, wg_grid(wgs), dim3(DL_THREADS), 0, st, x, (int)M, (int)K, w, (int)N, bias, y,
                            (int)mt, (int)nt, (int)wgs);
