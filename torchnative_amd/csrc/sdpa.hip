@@ -732,13 +732,13 @@ constexpr int PF_BQ = 16 * PF_WAVES, PF_BK = 64;
 // products times |scale|. us on the plain kernel -> here: 4 heads, 1024 causal keys, head
 // dim 96: 518 -> 57.5; 2 x 8 heads, 200 queries, 1000 keys, head dim 72: 667 -> 38;
 // 2 x 8 heads, 300 causal keys, head dim 256: 481 -> 45.
-template <int D, int BK, int MASK = 0, bool ANY = false>
+template <int D, int BK, int MASK = 0, bool ANY = false, bool AHEAD = false>
 __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__ Qg, const float* __restrict__ Kg,
                                               const float* __restrict__ Vg, int Hq, int Hkv, int L, int S,
                                               float sl2, int causal, const SkGeo geo,
                                               float* __restrict__ Og, float* __restrict__ lse,
                                               float* __restrict__ part_o, float2* __restrict__ part_ml,
-                                              uint32_t* __restrict__ tickets, const MaskRef mask, int mahead, int Dr, float qsign) {
+                                              uint32_t* __restrict__ tickets, const MaskRef mask, int Dr, float qsign) {
     constexpr int BQ = PF_BQ;
     const int DM = ANY ? Dr : D;  // the head dim in memory
     constexpr int RS = D + 4;
@@ -792,6 +792,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                 for (int i = 0; i < 4; i++) o[e][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
             float m = -INFINITY, l = 0.0f;
 
+            // AHEAD: a tile's mask quads requested with it (MaskAhead)
             using MA = MaskAhead<MASK == 0 ? 3 : MASK, false>;
             [[maybe_unused]] const MA ma(mask, b, h, qi, L, S);
             [[maybe_unused]] typename MA::quad mq[BK / 16];
@@ -832,11 +833,9 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                 const int buf = (t - t_begin) & 1;
                 const int k0 = t * BK;
                 // before the next tile's K and V: waiting for it leaves those in flight
-                if constexpr (MASK != 0) {
-                    if (mahead) {
+                if constexpr (AHEAD) {
         #pragma unroll
-                        for (int kt = 0; kt < BK / 16; kt++) mq[kt] = ma.load(k0 + 16 * kt + 4 * g);
-                    }
+                    for (int kt = 0; kt < BK / 16; kt++) mq[kt] = ma.load(k0 + 16 * kt + 4 * g);
                 }
                 if (t + 1 < t_end) gload(k0 + BK);
 
@@ -863,7 +862,7 @@ __global__ __launch_bounds__(PF_THREADS) void k_fa_f32(const float* __restrict__
                 }
                 if constexpr (MASK != 0) {
                     // scores to log2 units with the mask added; from here on the scale is 1
-                    if (mahead) {
+                    if constexpr (AHEAD) {
         #pragma unroll
                         for (int kt = 0; kt < BK / 16; kt++) {
                             const f32x4 mv = ma.values(mq[kt]);
@@ -2361,6 +2360,25 @@ tn_status flash_plan(hipStream_t st, int64_t B, int64_t Hq, int64_t L, int64_t S
 
 using namespace tn;
 
+// Whether an f32 call at a small head dim stays on the plain kernel, in tenths of a
+// microsecond beyond a launch. That one takes 32 rows a workgroup, one workgroup a
+// CU, key tiles of 32 at 1.2 us and as much for each 8 columns; the padded kernel's
+// tiles are 64 keys and 64 columns whatever the head dim (5 us), and the blocks that
+// its even split cuts are merged. Measured, us, plain / padded: 4 heads of 7 x 16, D
+// 8 5.4/8.1, D 16 6.7/8.3, D 24 8.0/8.3, D 32 9.3/8.3; 128 x 128, D 8 12.9/13.1, D 12
+// 17.9/13.4; 256 heads of 1 x 200, D 8 20.2/24.8, D 16 28.8/24.9; 1 x 64 8.2/8.3,
+// 10.7/8.4.
+static bool plain_f32(int64_t BH, int64_t L, int64_t S, int64_t D, bool masked) {
+    if (D > 24) return false;
+    const int64_t plain =
+        cdiv(BH * cdiv(L, ANY_BQ), 256) * cdiv(S, 32) * (12 * (cdiv(D, 8) + 1) + (masked ? 10 : 0));
+    const int64_t tiles = cdiv(S, 64), units = BH * cdiv(L, PF_BQ) * tiles;
+    const int64_t padded = tiles == 1     ? 50 + 43 * (cdiv(units, 256) - 1)
+                           : units <= 256 ? 80 + std::min<int64_t>(L, PF_BQ) / 6
+                                          : 55 + 83 * cdiv(units, 512);
+    return plain <= padded;
+}
+
 // The f32 flash kernel. any: head dims other than 64 and 128 and scales of at
 // most zero, on the padded variants; there *taken is false, and nothing was launched, where
 // a capture could not grow the stream's buffers.
@@ -2417,17 +2435,19 @@ static tn_status flash_f32(hipStream_t st, bool any, const void* q, const void* 
         const int me = mk == 1 ? 4 : 1;
         const bool quads = mref.sk == 1 && S % 4 == 0 && mref.sl % 4 == 0 && mref.sh % 4 == 0 && mref.sb % 4 == 0 &&
                            reinterpret_cast<uintptr_t>(mref.p) % (4 * me) == 0;
-        const int ahead = mahead && !quads;
+        const bool ahead = mahead && !quads;
         // an f32 query takes an f32 mask (mk 1) or a bool one (mk 3)
-#define TN_FA(DD, BKK, MK, ANY)                                                                                  \
-    hipLaunchKernelGGL((k_fa_f32<DD, BKK, MK, ANY>), dim3((unsigned)geo.G), dim3(PF_THREADS), 0, st, qq, kk, vv,      \
+#define TN_FA(DD, BKK, MK, ANY, AH)                                                                              \
+    hipLaunchKernelGGL((k_fa_f32<DD, BKK, MK, ANY, AH>), dim3((unsigned)geo.G), dim3(PF_THREADS), 0, st, qq, kk, vv, \
                        (int)Hq, (int)Hkv, (int)L, (int)S, asl2, c, geo, oo, lse, part_o, part_ml, tick, mref,   \
-                       ahead, (int)D, qsign)
-#define TN_FA_MK(DD, BKK, ANY)                \
-    do {                                      \
-        if (mk == 1) TN_FA(DD, BKK, 1, ANY);  \
-        else if (mk == 3) TN_FA(DD, BKK, 3, ANY); \
-        else TN_FA(DD, BKK, 0, ANY);          \
+                       (int)D, qsign)
+#define TN_FA_MK(DD, BKK, ANY)                               \
+    do {                                                     \
+        if (mk == 1 && ahead) TN_FA(DD, BKK, 1, ANY, true);  \
+        else if (mk == 1) TN_FA(DD, BKK, 1, ANY, false);     \
+        else if (mk == 3 && ahead) TN_FA(DD, BKK, 3, ANY, true); \
+        else if (mk == 3) TN_FA(DD, BKK, 3, ANY, false);     \
+        else TN_FA(DD, BKK, 0, ANY, false);                  \
     } while (0)
         // at most zero only if any; a zero scale makes q zeros, as hidden keys'
         // -inf is not to be multiplied by it
@@ -2549,7 +2569,8 @@ tn_status tn_sdpa_fwd(void* stream, int dtype, const void* q, const void* k, con
             }
         }
         if (dtype == TN_F32 && D % 4 == 0 &&
-            ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0) {
+            ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) % 16 == 0 &&
+            !plain_f32(B * Hq, L, S, D, mk != 0)) {
             bool taken = false;
             TN_TRY(flash_f32(st, true, q, k, v, B, Hq, Hkv, L, S, D, sl2, c, mk, mref, mahead, out, lse, &taken));
             if (taken) return TN_OK;
