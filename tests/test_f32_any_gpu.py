@@ -43,7 +43,8 @@ def _inputs(tn, B, Hq, Hkv, L, S, D, seed):
     # B, Hq, Hkv, L, S, D
     (1, 1, 1, 1, 1, 4), (2, 2, 1, 127, 63, 20), (1, 2, 2, 129, 65, 36), (1, 2, 2, 128, 64, 60), (1, 3, 1, 130, 33, 72),
     (2, 4, 2, 100, 300, 96), (1, 2, 1, 260, 260, 124), (1, 2, 2, 65, 17, 132), (1, 2, 1, 140, 140, 256),
-    (1, 1, 1, 5, 3000, 80), (3, 4, 1, 300, 300, 32), (1, 2, 2, 64, 64, 30)])  # 30: the plain kernel
+    (1, 1, 1, 5, 3000, 80), (3, 4, 1, 300, 300, 32), (1, 2, 2, 64, 64, 30),
+    (1, 1, 1, 1, 1, 32), (1, 2, 1, 130, 200, 4)])  # the plain kernel: head dims 30, and 4 over one key
 @pytest.mark.parametrize("causal", [False, True])
 def test_rows_keys_and_head_dims(tn, shape, causal):
     (q, k, v), w = _inputs(tn, *shape, seed=sum(shape))

@@ -157,17 +157,17 @@ def test_default_scale_and_explicit_scale_agree(tn):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
-def test_negative_scale_runs_on_the_plain_kernel(tn, dtype):
-    """The MFMA kernels take the row maximum of the unscaled scores, right
-    only for scale >= 0; a negative scale runs on the plain kernel, whose
-    maximum is over the scaled scores."""
+def test_negative_scale(tn, dtype):
+    """The kernels for head dims 64 and 128 take the row maximum of the
+    unscaled scores, right only for a positive scale; a negative one runs on
+    the kernels for any head dim, whose maximum is over the scaled scores."""
     q, k, v = _det((1, 4, 70, 64), 41), _det((1, 2, 90, 64), 42), _det((1, 2, 90, 64), 43)
     _check(tn, dtype, q, k, v, True, scale=-0.125)
     _check(tn, dtype, q, k, v, False, scale=-0.3)
 
 
 ANY_SHAPES = [
-    # head dims the MFMA kernels do not take: the plain kernel
+    # head dims other than 64 and 128 (1: the plain kernel, the others on the matrix cores)
     (1, 4, 2, 40, 70, 32),
     (2, 3, 1, 33, 50, 80),
     (1, 6, 3, 17, 29, 72),
@@ -284,8 +284,9 @@ def test_decode_f16_caches(tn):
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16", "float32"])
 def test_decode_other_head_dims(tn, dtype):
-    """Head dims the MFMA decode kernels do not take run on the plain kernel,
-    with ragged lengths, an empty sequence and truncation at max_len."""
+    """Head dims other than 64 and 128, with ragged lengths, an empty sequence
+    and truncation at max_len (head dims that stay on the plain kernel:
+    test_plain_attention_gpu.py)."""
     _decode_case(tn, 3, 8, 2, 96, [1, 77, 300], 320, 71, dtype=dtype)
     _decode_case(tn, 3, 4, 4, 32, [0, 5, 40], 48, 72, dtype=dtype)
     _decode_case(tn, 2, 6, 3, 80, [100, 50], 128, 73, max_len=64, dtype=dtype)
