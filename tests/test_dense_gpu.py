@@ -131,6 +131,22 @@ def test_reduced_formats_store_half_narrowing_and_widen_exactly(tn, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
+def test_narrowing_over_every_exponent(tn, fmt):
+    """Both signs of every f32 exponent, subnormals and NaNs included, with
+    mantissas at random, at the format's ties and one off them."""
+    rng = np.random.default_rng(22)
+    drop = 13 if fmt == "f16" else 16
+    m = rng.integers(0, 1 << 23, size=(512, 256), dtype=np.uint32)
+    tie = (m[:, :64] >> drop << drop) | (1 << (drop - 1))
+    m[:, :64], m[:, 64:96], m[:, 96:128] = tie, tie[:, :32] - 1, tie[:, 32:] + 1
+    bits = (np.arange(512, dtype=np.uint32)[:, None] << 23) | m
+    q = tn._quantize(_dev(tn, bits.view(np.float32)), fmt)
+    got = np.frombuffer(tn._quantized_blob(q), np.uint16).reshape(512, 256)
+    want = (O.f16_from_f32 if fmt == "f16" else O.bf16_from_f32)(bits.view(np.float32))
+    assert np.array_equal(got, want.reshape(512, 256))
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
 def test_a_signalling_nan_from_a_blob_widens_quieted(tn, fmt):
     h = np.array([0x7C01, 0xFC01, 0x7E00, 0x3C00] if fmt == "f16" else [0x7F81, 0xFF81, 0x7FC0, 0x3F80],
                  np.uint16).repeat(8).reshape(1, 32)
