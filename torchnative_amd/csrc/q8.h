@@ -49,9 +49,9 @@ __device__ inline void load_x8<uint16_t>(const uint16_t* p, float (&v)[8]) {
 }
 
 // The Q8_0 codes of one block held by four lanes, eight elements each: the
-// block's amax (order-free), d = amax/127, id = 1/d and the rounding are
-// q8_0_lane's, element for element, so the codes, the scale and the code sum
-// are identical; the sum comes back through `s`.
+// block's amax (order-free), d = amax/127, id = 1/d (the f32 d, not the stored
+// f16 one), codes rounded half away from zero (BlockQ8_0::from_float,
+// k_quants.rs:676-705); the code sum comes back through `s`.
 __device__ inline void q8_0_quad(const float (&v)[8], int (&q)[8], float* dx, int* s) {
     float a = 0.0f;  // f32::max from 0: NaNs are skipped (k_quants.rs:676-705)
 #pragma unroll

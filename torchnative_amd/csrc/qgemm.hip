@@ -30,9 +30,11 @@
 // What bounds it: the recurrence's 16 VALU instructions per tile and block
 // (convert, two products, a sum, four elements each), issued every 4.3 cycles
 // by a SIMD with several waves and every 8 by one with a single wave. 2 x 2 tiles
-// run at 72 cycles a tile and block ([512, 4096] x [14336, 4096] in 123 us, 490
-// TFLOP/s), one tile at 110 (17.9 us at m = 16, where a SIMD has one wave; the
-// prepass is 4 us of that).
+// take about 33 ns a tile and block on each SIMD, 78 cycles at 2.4 GHz, of which
+// those 16 are 69 ([512, 4096] x [14336, 4096] in 124 us, 485 TFLOP/s, 5-7 of it the
+// prepass). One tile a wave, alone on its SIMD, takes 110 ns, some 260 cycles (14.3
+// of the 17.8 us at m = 16; the prepass is 4): 128 are the 16, the rest the scale's
+// widening, the nibbles, the LDS reads and the waits, not measured one by one.
 //
 // Compared and not kept: two waves rounding two rows each of the same products
 // (23 us at m = 16: the doubled reads cost what the halved roundings saved); 4 x 2
