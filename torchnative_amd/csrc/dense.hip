@@ -461,7 +461,7 @@ __global__ void __launch_bounds__(DL_THREADS) k_dense_valu(const float* __restri
 //   1760 [1000, K] x [7000, K]: K 24 17.9/23.8  40 20.6/25.5  48 22.6/20.9   f16: 40 22.0/21.0
 inline bool dense_valu(int64_t M, int64_t N, int64_t K, bool lds, bool f32) {
     const int64_t wgs = cdiv(M, DV_T) * cdiv(N, DV_T);
-    if (wgs <= 128 || K < 8) return false;
+    if (wgs <= 128 || K < 8 || cdiv(N, DV_T) > WG_ROW) return false;  // (its grid has the features in x alone)
     if (lds) {
         if (wgs <= 256 || K >= 64) return false;
         if (wgs < 512) return K < 48;
